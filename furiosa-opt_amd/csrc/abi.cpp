@@ -982,6 +982,9 @@ int32_t fo_runtime_init(int32_t device_index, fo_runtime** out) {
       FO_HIP(hipGetDeviceProperties(&prop, device_index));
       rt->cus = prop.multiProcessorCount;
       rt->arch = prop.gcnArchName;
+      FO_HIP(hipMalloc((void**)&rt->gemm_ws.parts, fo::GemmWorkspace::kBytes));
+      FO_HIP(hipMalloc((void**)&rt->gemm_ws.arrived, fo::GemmWorkspace::kTiles * sizeof(uint32_t)));
+      launch_zero(rt->stream, rt->gemm_ws.arrived, fo::GemmWorkspace::kTiles * sizeof(uint32_t));
       const char* eager = getenv("FO_EAGER");
       rt->eager = eager && *eager && std::strcmp(eager, "0") != 0;
     } catch (...) {
@@ -1028,6 +1031,8 @@ void fo_runtime_free(fo_runtime* rt) {
   }
   if (rt->trace_base) (void)hipEventDestroy(rt->trace_base);
   if (rt->scratch) (void)hipFree(rt->scratch);
+  if (rt->gemm_ws.parts) (void)hipFree(rt->gemm_ws.parts);
+  if (rt->gemm_ws.arrived) (void)hipFree(rt->gemm_ws.arrived);
   if (rt->pool) {
     std::lock_guard<std::mutex> lock(rt->pool->mu);
     for (auto& kv : rt->pool->cached) (void)hipFree(kv.second);
@@ -2227,7 +2232,7 @@ void contraction_impl(fo_runtime* rt, fo_buffer* out, const fo_buffer* lhs, cons
           int64_t amax = (d.batch - 1) * d.a_batch + (d.M - 1) * d.lda + d.K - 1;
           int64_t bmax = (d.batch - 1) * d.b_batch + (d.N - 1) * d.ldb + d.K - 1;
           if (amax < lhs_len && bmax < rhs_len && gemm_aligned(L, R, ct, d)) {
-            launch_gemm(rt->stream, O, L, R, ct, co, d);
+            launch_gemm(rt->stream, O, L, R, ct, co, d, rt->gemm_ws);
             return;
           }
         }
@@ -2403,7 +2408,7 @@ int32_t fo_gemm_w8a8_dequant(fo_runtime* rt, fo_buffer* out, fo_buffer* acc_out,
     set_device(rt);
     TraceScope trace_span(rt, "gemm_w8a8_dequant");
     launch_w8a8(rt->stream, (uint16_t*)out->ptr, acc_out ? (int32_t*)acc_out->ptr : nullptr, (const int8_t*)a->ptr,
-                (const int8_t*)w->ptr, (const float*)scale->ptr, m, n, k);
+                (const int8_t*)w->ptr, (const float*)scale->ptr, m, n, k, rt->gemm_ws);
   });
 }
 

@@ -6,7 +6,7 @@
 // Tiling (gfx950, wave64): a block of WM x WN waves owns a BM x BN tile; each wave owns
 // (BM/WM) x (BN/WN) as a grid of 32x32 MFMA tiles (v_mfma_f32_32x32x16_bf16 /
 // v_mfma_i32_32x32x32_i8 / v_mfma_f32_32x32x64_f8f6f4 for the two 8-bit float formats, OCP E4M3
-// and E5M2, the encodings of f8e4m3 / f8e5m2). K advances kRB bytes per stage; kNS stages rotate
+// and E5M2, the encodings of f8e4m3 / f8e5m2). K advances kRB bytes per stage; NS stages rotate
 // through LDS. The
 // DMA refilling a buffer is issued right after the barrier that releases it, and each stage waits
 // only for its own DMA (vmcnt counts the younger ones).
@@ -25,6 +25,7 @@
 // k -> (lane, element) map, and the sum over k is order-free up to f32 rounding (exact for i32).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "runtime.hpp"
@@ -41,7 +42,6 @@ typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2_t;
 typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8_t;
 
 constexpr int kRB = 128;  // K bytes per row per stage (four 32-byte MFMA k-steps)
-constexpr int kNS = 2;    // LDS stages (double buffer; 64-byte stages x4 measured slower: more barriers)
 constexpr int kCPR = kRB / 16;                  // 16-byte chunks per row
 constexpr int kRPC = 1024 / kRB;                // rows per 1 KiB wave DMA
 constexpr int kSwzShift = kRB == 64 ? 2 : 1;    // rows sharing a bank-group offset: 16 / kCPR
@@ -105,6 +105,9 @@ struct GemmArgs {
   int64_t lda, ldb, ldc_m, ldc_n;  // elements
   int64_t a_batch, b_batch, c_batch;
   int32_t tiles_m, tiles_n;
+  int32_t splits;      // blocks sharing an output tile, each a run of k stages (k_gemm; 1: none)
+  uint64_t* parts;     // splits > 1: partial accumulators
+  uint32_t* arrived;   // splits > 1: blocks of each tile that have stored theirs (zero between launches)
   const float* scale;  // OUT == 4: per-column dequant scale
   int32_t* acc_out;    // OUT == 4: optional raw i32 accumulators (row-major, ldc_m / ldc_n)
 };
@@ -190,7 +193,52 @@ __device__ __forceinline__ i32x4_t regroup8(i32x2_t a, i32x2_t b) {
   return i32x4_t{(int)r0[0], (int)r1[0], (int)r0[1], (int)r1[1]};
 }
 
-template <int KIND, int OUT, int BM, int BN, int WM, int WN>
+// The partial accumulators of a tile's blocks, summed by the last of them to arrive (in split order,
+// so the result does not depend on which block that is). True for that block, with the sums in acc.
+// Partials and the arrival count go through agent-scope accesses, which bypass the per-XCD L2s'
+// private copies; each block's stores have completed (vmcnt 0 in every wave, then the barrier)
+// before its arrival is counted. The last block zeroes the count for the next launch.
+template <int TILES, int THREADS, typename A>
+__device__ __forceinline__ bool combine_splits(const GemmArgs& g, int tile, int split, A* acc) {
+  constexpr int Q = 8;  // 64-bit words per accumulator tile and lane
+  const int tid = threadIdx.x;
+  uint64_t* base = g.parts + (int64_t)tile * g.splits * (TILES * Q * THREADS) + tid;
+  uint64_t* own = base + (int64_t)split * (TILES * Q * THREADS);
+#pragma unroll
+  for (int t = 0; t < TILES; ++t)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      // Copies: a bit cast of a vector element itself reads element 0.
+      const auto a0 = acc[t][2 * q], a1 = acc[t][2 * q + 1];
+      const uint32_t lo = __builtin_bit_cast(uint32_t, a0), hi = __builtin_bit_cast(uint32_t, a1);
+      __hip_atomic_store(own + (t * Q + q) * THREADS, (uint64_t)lo | (uint64_t)hi << 32, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
+  __shared__ uint32_t order;
+  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) order = __hip_atomic_fetch_add(g.arrived + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (order != (uint32_t)g.splits - 1) return false;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  if (tid == 0) __hip_atomic_store(g.arrived + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int s = 0; s < g.splits; ++s) {
+    const uint64_t* p = base + (int64_t)s * (TILES * Q * THREADS);
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const uint64_t w = __hip_atomic_load(p + (t * Q + q) * THREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const auto lo = __builtin_bit_cast(decltype(acc[0][0] + 0), (uint32_t)w);
+        const auto hi = __builtin_bit_cast(decltype(acc[0][0] + 0), (uint32_t)(w >> 32));
+        acc[t][2 * q] = s ? acc[t][2 * q] + lo : lo;
+        acc[t][2 * q + 1] = s ? acc[t][2 * q + 1] + hi : hi;
+      }
+  }
+  return true;
+}
+
+template <int KIND, int OUT, int BM, int BN, int WM, int WN, int NS>
 __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   using M = MfmaT<KIND>;
   using acc_t = typename M::acc_t;
@@ -215,7 +263,8 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   // Tile order: consecutive block ids go round-robin over the 8 XCDs; regroup so each XCD walks a
   // contiguous range of tiles, ordered in groups of 8 tile-rows so neighbours share operands in L2.
   const int ntiles = g.tiles_m * g.tiles_n;
-  int bid = blockIdx.x;
+  const int split = (int)blockIdx.x / ntiles;  // 0 when splits == 1
+  int bid = (int)blockIdx.x - split * ntiles;
   int tile = bid;
   if ((ntiles % 8) == 0) tile = (bid % 8) * (ntiles / 8) + bid / 8;
   const int group = 8;
@@ -233,6 +282,10 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   const int wm = wave / WN, wn = wave % WN;
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
   const uint32_t KB = (uint32_t)(g.K * EB);  // K in bytes
+  // This block's k stages: [st0, st0 + nst) of the contraction's.
+  const int nst_all = (int)((KB + kRB - 1) / kRB);
+  const int st0 = (int)((int64_t)nst_all * split / g.splits);
+  const int nst = (int)((int64_t)nst_all * (split + 1) / g.splits) - st0;
 
   // Buffer resources based at the tile's first row, extent = the bytes its valid rows span.
   const int64_t rows_a = min((int64_t)BM, g.M - m0), rows_b = min((int64_t)BN, g.N - n0);
@@ -266,8 +319,8 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   // constant at every (inlined) call.
   auto issue_rng = [&](int st, int lo, int hi, bool FULL) __attribute__((always_inline)) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass drops the kernel stubs over these builtins
-    const uint32_t kb = (uint32_t)st * kRB;
-    const int buf = st % kNS;
+    const uint32_t kb = (uint32_t)(st0 + st) * kRB;
+    const int buf = st % NS;
     const bool tail = !FULL && kb + kRB > KB;  // uniform
 #pragma unroll
     for (int i = 0; i < A_CH; ++i) {
@@ -312,7 +365,6 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   const int a_row = (wm * TWM + frow) * kRB, b_row = (wn * TWN + frow) * kRB;
   auto slot = [&](int kk, int e) { return (((KSTEP / 16) * kk + (FRAG / 16) * half + e) ^ swz) * 16; };
 
-  const int nst = (int)((KB + kRB - 1) / kRB);
   constexpr int KST = kRB / KSTEP;  // MFMA k-steps per stage
   static_assert(KST % 2 == 0, "fragment double-buffer parity assumes an even k-step count");
   // Stage s's DMA is complete once at most the younger stages' DMAs are outstanding; after the
@@ -320,9 +372,9 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   // so that stage's buffer can be refilled. The barrier carries no memory fence (that would drain
   // every DMA); the compiler barriers keep LDS accesses on their side of it.
   auto stage_ready = [&](int s) {
-    // DMAs in flight younger than stage s: the prologue fills all kNS buffers; afterwards the
-    // refill of stage s - 1's buffer (stage s - 1 + kNS) is issued after this barrier.
-    const int ahead = min(nst - 1 - s, s == 0 ? kNS - 1 : kNS - 2);
+    // DMAs in flight younger than stage s: the prologue fills all NS buffers; afterwards the
+    // refill of stage s - 1's buffer (stage s - 1 + NS) is issued after this barrier.
+    const int ahead = min(nst - 1 - s, s == 0 ? NS - 1 : NS - 2);
     if (ahead >= 3)
       __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(3 * PER));
     else if (ahead == 2)
@@ -362,7 +414,7 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   };
 
 #pragma unroll
-  for (int st = 0; st < kNS; ++st)
+  for (int st = 0; st < NS; ++st)
     if (st < nst) issue_rng(st, 0, PER, false);
   stage_ready(0);
   read_frags(0, 0, 0);
@@ -384,33 +436,35 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
     for (int kk = 0; kk < KST; ++kk) {
       const int p = kk & 1;  // KST is even: the fragment buffer parity restarts each stage
       if (kk + 1 < KST) {
-        read_frags(s % kNS, kk + 1, p ^ 1);
-        const int r = s + kNS - 1;  // refilled after stage s - 1's last barrier
-        if (kk + 1 < NP && (S || (r >= kNS && r < nst)))
+        read_frags(s % NS, kk + 1, p ^ 1);
+        const int r = s + NS - 1;  // refilled after stage s - 1's last barrier
+        if (kk + 1 < NP && (S || (r >= NS && r < nst)))
           issue_rng(r, (kk + 1) * PER / NP, (kk + 2) * PER / NP, S);
       } else if (S || s + 1 < nst) {
         __builtin_amdgcn_sched_barrier(0);
         stage_ready(s + 1);
         __builtin_amdgcn_sched_barrier(0);
-        read_frags((s + 1) % kNS, 0, p ^ 1);
+        read_frags((s + 1) % NS, 0, p ^ 1);
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = M::mma(fb[p][j], fa[p][i], acc[i][j]);
       __builtin_amdgcn_iglp_opt(0);  // interleave the fragment reads with the MFMAs
-      if (kk + 1 == KST && (S || s + kNS < nst)) {
+      if (kk + 1 == KST && (S || s + NS < nst)) {
         __builtin_amdgcn_sched_barrier(0);
-        issue_rng(s + kNS, 0, PER / NP, S);
+        issue_rng(s + NS, 0, PER / NP, S);
       }
     }
   };
-  // Steady stages: s >= 1 (the prologue issued stages 0 .. kNS - 1) and s + kNS <= nst - 2 (every
+  // Steady stages: s >= 1 (the prologue issued stages 0 .. NS - 1) and s + NS <= nst - 2 (every
   // stage they refill lies before the last, the only one that may be partial).
   int s = 0;
   if (nst > 0) stage(s++, false);
-  for (; s + kNS + 2 <= nst; ++s) stage(s, true);
+  for (; s + NS + 2 <= nst; ++s) stage(s, true);
   for (; s < nst; ++s) stage(s, false);
+
+  if (g.splits > 1 && !combine_splits<TM * TN, 64 * W>(g, batch * ntiles + tile, split, &acc[0][0])) return;
 
   // Epilogue. With B as the MFMA's A operand, lane holds row m = 32i + (lane % 32) of the wave
   // tile and columns n = 32j + 8*(v/4) + 4*(lane/32) + v%4: four consecutive columns per v / 4.
@@ -900,9 +954,8 @@ __global__ void __launch_bounds__(256, 1) k_gemm4(GemmArgs g) {
   });
 }
 
-template <int KIND, int OUT, int NSA>
-void gemm4_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, const void* b, const float* scale,
-                      int32_t* acc_out) {
+GemmArgs gemm_args(const GemmDesc& d, void* c, const void* a, const void* b, const float* scale, int32_t* acc_out,
+                   int bm, int bn) {
   GemmArgs g;
   g.a = (const uint8_t*)a;
   g.b = (const uint8_t*)b;
@@ -917,10 +970,20 @@ void gemm4_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, 
   g.a_batch = d.a_batch;
   g.b_batch = d.b_batch;
   g.c_batch = d.c_batch;
+  g.splits = 1;
+  g.parts = nullptr;
+  g.arrived = nullptr;
   g.scale = scale;
   g.acc_out = acc_out;
-  g.tiles_m = (int)((d.M + 255) / 256);
-  g.tiles_n = (int)((d.N + 255) / 256);
+  g.tiles_m = (int)((d.M + bm - 1) / bm);
+  g.tiles_n = (int)((d.N + bn - 1) / bn);
+  return g;
+}
+
+template <int KIND, int OUT, int NSA>
+void gemm4_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, const void* b, const float* scale,
+                      int32_t* acc_out) {
+  const GemmArgs g = gemm_args(d, c, a, b, scale, acc_out, 256, 256);
   const size_t lds = (size_t)(NSA + 2) * 256 * 128;
   static bool attr_set = false;
   if (!attr_set) {
@@ -933,72 +996,77 @@ void gemm4_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, 
   FO_HIP(hipGetLastError());
 }
 
-template <int KIND, int OUT, int BM, int BN, int WM, int WN>
+template <int KIND, int OUT, int BM, int BN, int WM, int WN, int NS>
 void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, const void* b, const float* scale,
-                     int32_t* acc_out) {
-  GemmArgs g;
-  g.a = (const uint8_t*)a;
-  g.b = (const uint8_t*)b;
-  g.c = c;
-  g.M = d.M;
-  g.N = d.N;
-  g.K = d.K;
-  g.lda = d.lda;
-  g.ldb = d.ldb;
-  g.ldc_m = d.ldc_m;
-  g.ldc_n = d.ldc_n;
-  g.a_batch = d.a_batch;
-  g.b_batch = d.b_batch;
-  g.c_batch = d.c_batch;
-  g.scale = scale;
-  g.acc_out = acc_out;
-  g.tiles_m = (int)((d.M + BM - 1) / BM);
-  g.tiles_n = (int)((d.N + BN - 1) / BN);
-  size_t lds = (size_t)kNS * (BM + BN) * kRB;
+                     int32_t* acc_out, int splits = 1, const GemmWorkspace* ws = nullptr) {
+  GemmArgs g = gemm_args(d, c, a, b, scale, acc_out, BM, BN);
+  const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
+  if (splits > 1) {
+    g.splits = splits;
+    g.parts = ws->parts;
+    g.arrived = ws->arrived;
+  }
+  constexpr size_t lds = (size_t)NS * (BM + BN) * kRB;
   static bool attr_set = false;  // gfx950 LDS is 160 KiB; dynamic LDS above 64 KiB must be opted into
   if (!attr_set) {
-    FO_HIP(hipFuncSetAttribute((const void*)k_gemm<KIND, OUT, BM, BN, WM, WN>,
+    FO_HIP(hipFuncSetAttribute((const void*)k_gemm<KIND, OUT, BM, BN, WM, WN, NS>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_set = true;
   }
-  dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)d.batch);
-  hipLaunchKernelGGL((k_gemm<KIND, OUT, BM, BN, WM, WN>), grid, dim3(64 * WM * WN), lds, s, g);
+  dim3 grid((unsigned)(tiles * splits), (unsigned)d.batch);
+  hipLaunchKernelGGL((k_gemm<KIND, OUT, BM, BN, WM, WN, NS>), grid, dim3(64 * WM * WN), lds, s, g);
   FO_HIP(hipGetLastError());
 }
 
-// Tile choice: 256x256 when the problem is large -- four waves of 128x128 in 16x16 MFMA tiles
-// (k_gemm4) for bf16 and i8 (plain outputs and the W8A8 dequant), eight waves of 128x64 in 32x32
-// tiles (k_gemm) for the 8-bit floats -- and 128x128 otherwise. FO_GEMM_TILE overrides it for
-// measurement: 128, 256 (k_gemm, 4 waves of 128x128), 2568 (8 waves of 128x64), 25616 (16 waves)
-// or 4128 (k_gemm4).
+// Tile choice, by how many tiles of each size the output has (T64, T128, T256; batches included)
+// on the 256 CUs. Measured on one box as the kernel alone in a recorded graph, bf16 -> bf16, us:
+//     M, N, K            64x64   128x128 4 stages   128x128 2 stages   256x256 (k_gemm4)
+//     500, 3072, 1024     10.0        12.9               15.3               38
+//     512, 4096, 4096     30.7        32.3               42.6               75      T64 = 512
+//     1024, 4096, 4096    58          42.5               48.1               76      T128 = 256
+//     2048, 4096, 4096   107          78.6               69.8               79      T128 = 512
+//     3000, 3000, 2992   140          92.6               95.6               81      T256 = 144
+//     2048, 8192, 1024    68          54                 44.8               37.5    T256 = 256
+// and the same order for i8. Hence: 64x64 (32 KiB of LDS a stage pair, two blocks a CU) up to two
+// tiles a CU; 128x128 with four stages in flight while one block a CU covers them; with two stages,
+// two blocks a CU, up to 512; past that 256x256: four waves of 128x128 in 16x16 MFMA tiles (k_gemm4)
+// for bf16 and i8, eight waves of 128x64 in 32x32 tiles (k_gemm) for the 8-bit floats, whose 32-byte
+// fragments have no 16x16 form here.
+//
+// Few 64x64 tiles leave CUs idle while each walks all of K, so up to 8 blocks share a tile while
+// that adds no second block to a CU and leaves each at least 12 stages (combine_splits costs about
+// 2.5 us): 64, 1024, 4096 in 10.6 us with 4 against 18.3 with one; 256, 256, 8192 in 13.2 with 8
+// against 32.7; with 8 stages left a split measured slower (16, 1024, 1024: 7.9 against 7.2).
+// FO_GEMM_TILE overrides the tile for measurement: 64, 128, 1284 (128x128, four stages), 2568 (k_gemm,
+// 256x256) or 4128 (k_gemm4).
 template <int KIND, int OUT>
-void gemm_launch(hipStream_t s, const GemmDesc& d, void* c, const void* a, const void* b,
+void gemm_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, void* c, const void* a, const void* b,
                  const float* scale = nullptr, int32_t* acc_out = nullptr) {
   static int forced = [] {
     const char* e = getenv("FO_GEMM_TILE");
     return e ? atoi(e) : 0;
   }();
-  int64_t tiles256 = ((d.M + 255) / 256) * ((d.N + 255) / 256) * d.batch;
-  // Large problems: 8 waves of 128x64 for every kind: bf16 1-1.5% above 16 waves of 64x64 at
-  // 4096^3 (same boxes, 200-launch runs); the 8-bit floats' 32-byte fragments make 16 waves of
-  // 64x64 exceed 128 VGPRs and spill (1850 TFLOP/s against 367); i8 (the W8A8 config) 2175-2186
-  // against 2135-2142 TOP/s with the refill split in parts.
   constexpr bool k16 = (KIND == kBf16 || KIND == kI8) && OUT <= 4;  // kinds with a 16x16 MFMA form here
-  // Four waves of 128x128 for every kind with a 16x16 form: bf16 1258-1273 (eight-wave) against 1319
-  // TFLOP/s, i8 -> i32 1660 against 1930 TOP/s, the W8A8 dequant 2432-2442 against 2490 TOP/s (same
-  // boxes; before the four-wave kernel's refill interleave the W8A8 measured the other way round).
-  constexpr bool k16_default = k16;
-  int choice = forced ? forced : (tiles256 >= 128 ? (k16_default ? 4128 : 2568) : 128);
+  auto tiles = [&](int64_t t) { return ((d.M + t - 1) / t) * ((d.N + t - 1) / t) * d.batch; };
+  const int64_t t64 = tiles(64);
+  int choice = forced;
+  if (!choice) choice = t64 <= 512 ? 64 : tiles(128) <= 256 ? 1284 : tiles(256) < 144 ? 128 : k16 ? 4128 : 2568;
   if constexpr (k16) {
     // four waves of 128x128 (16x16 MFMA tiles), 128-byte stages, A and B double-buffered. (A
     // triple-buffered, running a stage further ahead than B in the 32 KiB of LDS left over, measured
     // 1030-1034 against 1300-1307 TFLOP/s on one box: correct, and slower.)
     if (choice == 4128) return gemm4_launch_cfg<KIND, OUT, 2>(s, d, c, a, b, scale, acc_out);
   }
-  if (choice == 2568) return gemm_launch_cfg<KIND, OUT, 256, 256, 2, 4>(s, d, c, a, b, scale, acc_out);
-  if (choice == 25616) return gemm_launch_cfg<KIND, OUT, 256, 256, 4, 4>(s, d, c, a, b, scale, acc_out);
-  if (choice == 256) return gemm_launch_cfg<KIND, OUT, 256, 256, 2, 2>(s, d, c, a, b, scale, acc_out);
-  return gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2>(s, d, c, a, b, scale, acc_out);
+  if (choice == 64) {
+    const int64_t stages = (d.K * MfmaT<KIND>::EB + kRB - 1) / kRB;
+    int64_t splits = std::min<int64_t>({256 / std::max<int64_t>(t64, 1), stages / 12, 8});
+    if (splits < 1) splits = 1;
+    static_assert(GemmWorkspace::kTiles >= 256, "split workspace");
+    return gemm_launch_cfg<KIND, OUT, 64, 64, 2, 2, 4>(s, d, c, a, b, scale, acc_out, (int)splits, &ws);
+  }
+  if (choice == 1284) return gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 4>(s, d, c, a, b, scale, acc_out);
+  if (choice == 128) return gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 2>(s, d, c, a, b, scale, acc_out);
+  return gemm_launch_cfg<KIND, OUT, 256, 256, 2, 4, 2>(s, d, c, a, b, scale, acc_out);
 }
 
 }  // namespace
@@ -1017,22 +1085,22 @@ bool gemm_supported(fo_dtype in_t, fo_dtype out_t) {
 }
 
 void launch_gemm(hipStream_t s, void* c, const void* a, const void* b, fo_dtype in_t, fo_dtype out_t,
-                 const GemmDesc& d) {
+                 const GemmDesc& d, const GemmWorkspace& ws) {
   // 16-byte fragment loads need 16-byte aligned rows.
   require(gemm_aligned(a, b, in_t, d), "gemm: operands not 16-byte aligned or shape too large");
-  if (in_t == FO_BF16 && out_t == FO_BF16) return gemm_launch<kBf16, 0>(s, d, c, a, b);
-  if (in_t == FO_BF16 && out_t == FO_F32) return gemm_launch<kBf16, 1>(s, d, c, a, b);
-  if (in_t == FO_I8 && out_t == FO_I8) return gemm_launch<kI8, 2>(s, d, c, a, b);
-  if (in_t == FO_I8 && out_t == FO_I32) return gemm_launch<kI8, 3>(s, d, c, a, b);
-  if (in_t == FO_F8E4M3 && out_t == FO_F8E4M3) return gemm_launch<kF8E4M3, 5>(s, d, c, a, b);
-  if (in_t == FO_F8E4M3 && out_t == FO_F32) return gemm_launch<kF8E4M3, 1>(s, d, c, a, b);
-  if (in_t == FO_F8E5M2 && out_t == FO_F8E5M2) return gemm_launch<kF8E5M2, 6>(s, d, c, a, b);
-  if (in_t == FO_F8E5M2 && out_t == FO_F32) return gemm_launch<kF8E5M2, 1>(s, d, c, a, b);
+  if (in_t == FO_BF16 && out_t == FO_BF16) return gemm_launch<kBf16, 0>(s, d, ws, c, a, b);
+  if (in_t == FO_BF16 && out_t == FO_F32) return gemm_launch<kBf16, 1>(s, d, ws, c, a, b);
+  if (in_t == FO_I8 && out_t == FO_I8) return gemm_launch<kI8, 2>(s, d, ws, c, a, b);
+  if (in_t == FO_I8 && out_t == FO_I32) return gemm_launch<kI8, 3>(s, d, ws, c, a, b);
+  if (in_t == FO_F8E4M3 && out_t == FO_F8E4M3) return gemm_launch<kF8E4M3, 5>(s, d, ws, c, a, b);
+  if (in_t == FO_F8E4M3 && out_t == FO_F32) return gemm_launch<kF8E4M3, 1>(s, d, ws, c, a, b);
+  if (in_t == FO_F8E5M2 && out_t == FO_F8E5M2) return gemm_launch<kF8E5M2, 6>(s, d, ws, c, a, b);
+  if (in_t == FO_F8E5M2 && out_t == FO_F32) return gemm_launch<kF8E5M2, 1>(s, d, ws, c, a, b);
   throw InvalidArg("gemm: unsupported dtype pair");
 }
 
 void launch_w8a8(hipStream_t s, uint16_t* out, int32_t* acc_out, const int8_t* a, const int8_t* w, const float* scale,
-                 int64_t m, int64_t n, int64_t k) {
+                 int64_t m, int64_t n, int64_t k, const GemmWorkspace& ws) {
   GemmDesc d;
   d.M = m;
   d.N = n;
@@ -1042,7 +1110,7 @@ void launch_w8a8(hipStream_t s, uint16_t* out, int32_t* acc_out, const int8_t* a
   d.ldc_m = n;
   d.ldc_n = 1;
   require(gemm_aligned(a, w, FO_I8, d), "w8a8: k must be a multiple of 16 and operands 16-byte aligned");
-  gemm_launch<kI8, 4>(s, d, out, a, w, scale, acc_out);
+  gemm_launch<kI8, 4>(s, d, ws, out, a, w, scale, acc_out);
 }
 
 }  // namespace fo

@@ -55,8 +55,22 @@ struct fo_graph_mem {
   }
 };
 
+namespace fo {
+// Working memory of contractions whose blocks share output tiles (k_gemm with splits > 1): made with
+// the runtime, so no call allocates for it and recorded graphs may keep its address (graphs lose
+// their executables with their runtime). One call uses it at a time: the runtime's ops, launched
+// graphs included, run in order on its one stream.
+struct GemmWorkspace {
+  static constexpr int64_t kTiles = 256;                    // output tiles x blocks a tile of a split launch
+  static constexpr int64_t kBytes = kTiles * 64 * 64 * 4;  // their 64x64 partial accumulators
+  uint64_t* parts = nullptr;
+  uint32_t* arrived = nullptr;  // a counter per tile, zero between launches
+};
+}  // namespace fo
+
 struct fo_runtime {
   int device = 0;
+  fo::GemmWorkspace gemm_ws;
   std::shared_ptr<fo_pool> pool;
   hipStream_t stream = nullptr;
   hipEvent_t events[16] = {};
@@ -324,7 +338,7 @@ bool gemv_takes_f32_x(int64_t K);
 void launch_gemv(hipStream_t s, void* out, const void* x, const void* w, fo_dtype in_t, fo_dtype out_t, int64_t N,
                  int64_t K, int64_t ldw, int64_t ldo, bool x_f32 = false);
 void launch_gemm(hipStream_t s, void* c, const void* a, const void* b, fo_dtype in_t, fo_dtype out_t,
-                 const GemmDesc& d);
+                 const GemmDesc& d, const GemmWorkspace& ws);
 bool gemm_supported(fo_dtype in_t, fo_dtype out_t);
 bool gemm_aligned(const void* a, const void* b, fo_dtype in_t, const GemmDesc& d);
 
@@ -340,7 +354,7 @@ void launch_gemm_wheels(hipStream_t s, void* c, const void* a, const void* b, fo
 void launch_zero(hipStream_t s, void* p, uint64_t bytes);
 
 void launch_w8a8(hipStream_t s, uint16_t* out, int32_t* acc_out, const int8_t* a, const int8_t* w, const float* scale,
-                 int64_t m, int64_t n, int64_t k);
+                 int64_t m, int64_t n, int64_t k, const GemmWorkspace& ws);
 void launch_rmsnorm_softmax(hipStream_t s, uint16_t* out, const uint16_t* x, const uint16_t* gain, int64_t rows,
                             int64_t cols, float eps);
 void launch_attention_prefill(hipStream_t s, uint16_t* out, const uint16_t* q, const uint16_t* k, const uint16_t* v,
