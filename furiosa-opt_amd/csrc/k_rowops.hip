@@ -4,14 +4,14 @@
 // slice reduce; fp_div by the column count; clip Add eps; Sqrt; (x * g) / r in f32; cast to bf16 at
 // commit. The softmax re-fetches the committed bf16 values: max, exp(y - max), sum, divide, cast.
 //
-// Layout: lane l of a wave holds the 16-byte chunks c*64 + l of its part of the row (8 bf16 each), so
-// every wave load or store is 1 KiB contiguous. The row stays packed as bf16 in registers (x, then
-// y); exp(y - max) is held in f32 registers from the sum to the output, so each element is read,
-// exponentiated and written once. The gain is staged once per block in LDS as f32. Two kernels:
-//   * k_rmsnorm_softmax_dma (512 to 4096 columns): one wave per row, persistent waves, the next row
-//     fetched into LDS by DMA while the current one is computed;
-//   * k_rmsnorm_softmax_split (8192 columns): a row spread over four waves, whose reductions combine
-//     through LDS, so that a wave's registers still hold its share of the row and its exponentials.
+// Layout: a lane holds 16-byte chunks of its row (8 bf16 each), consecutive lanes consecutive chunks, so a
+// wave's load or store is 1 KiB contiguous. exp(y - max) is held in f32 registers from the sum to the
+// output, so each element is read, exponentiated and written once. Two kernels:
+//   * k_rmsnorm_softmax_row (up to 32768 columns, any row length): one to sixteen waves per row;
+//   * k_rmsnorm_softmax_dma (4096 columns, many rows): one wave per row, persistent waves, the next row
+//     fetched into LDS by DMA while the current one is computed, the gain staged once per block.
+// Bound by HBM when large (5.1-5.4 TB/s, what a large copy reaches) and by the launch and one memory
+// round trip when small.
 //
 // Numerics. This file is compiled with f32 denormals flushed (inputs and results, sign kept),
 // which is the reference's own numeric model: its bf16 widen and narrow flush every subnormal to a
@@ -120,7 +120,7 @@ __device__ void row_exact(uint16_t* __restrict__ orow, const uint16_t* __restric
   }
 }
 
-// Rows of up to 4096 columns: one wave per row, persistent waves, the next row fetched into LDS
+// Rows of 4096 columns: one wave per row, persistent waves, the next row fetched into LDS
 // by DMA (buffer_load ... lds) while the current one is computed. A register prefetch would not
 // stay in flight: with this row's stores also outstanding the compiler waits for every access
 // before touching the prefetched registers. Here the only wait on vector memory is explicit and
@@ -277,143 +277,142 @@ void rs_dma_launch(hipStream_t s, uint16_t* out, const uint16_t* x, const uint16
                      (float)(NCH * 512), eps);
 }
 
-// Split rows (8192 columns): a block of kSplit waves normalises one row at a time, each wave holding
-// CPW 16-byte chunks per lane (cols = kSplit * CPW * 512); the three row reductions combine the
-// waves' partials through LDS. Blocks are persistent and loop over rows; latency is hidden by the
-// other blocks on the CU (four waves per SIMD at CPW = 4) rather than by a prefetch.
-constexpr int kSplit = 4;
-template <int CPW>
-__global__ void __launch_bounds__(64 * kSplit) k_rmsnorm_softmax_split(uint16_t* __restrict__ out,
-                                                                      const uint16_t* __restrict__ x,
-                                                                      const uint16_t* __restrict__ gain, int64_t rows,
-                                                                      float cols_f, float eps) {
-  constexpr int cols = kSplit * CPW * 512;
+// A row of up to 32768 columns over W waves, P elements a lane held in registers from the load to the
+// output (x, then y, then exp(y - max)), so the row is read once. Element e of chunk c of thread t is
+// column (c * T + t) * 8 + e, T = 64 W. Chunks are 16-byte accesses at any even address (rows of an
+// odd length start anywhere); the row's last, partial chunk goes element by element. The gain is read
+// per row, from the caches.
+typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+typedef u16x8 u16x8_any __attribute__((aligned(2)));
+
+template <int P, int W, bool NT>
+__global__ void __launch_bounds__(W < 4 ? 256 : 64 * W) k_rmsnorm_softmax_row(uint16_t* __restrict__ out,
+                                                                         const uint16_t* __restrict__ x,
+                                                                         const uint16_t* __restrict__ gain, int64_t rows,
+                                                                         int cols, float eps) {
+  constexpr int NC = P / 8;
+  constexpr int T = 64 * W;
+  constexpr int R = W < 4 ? 4 / W : 1;  // rows per block
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-  __shared__ __attribute__((aligned(16))) float sg[cols];
-  __shared__ float red[3][kSplit];
-  __shared__ int g_bad;
-  if (threadIdx.x == 0) g_bad = 0;
-  __syncthreads();
-  // Gain staged once per block, widened by the reference rule; at or above 2^120 in magnitude it
-  // takes the exact path, as in k_rmsnorm_softmax_dma.
-  int bad_local = 0;
-  for (int i = threadIdx.x; i < cols; i += blockDim.x) {
-    float gv = bf16_to_f32(gain[i]);
-    sg[i] = gv;
-    bad_local |= !(__builtin_fabsf(gv) < 0x1p120f);
+  const int wave = (threadIdx.x >> 6) % W, slot = (threadIdx.x >> 6) / W;
+  const int64_t row = (int64_t)blockIdx.x * R + slot;
+  const bool live = row < rows;  // no early return: the barriers below are the block's
+  const int t = wave * 64 + lane;
+  __shared__ float red[3][R][W];
+  auto combine = [&](int k, float v, bool max) __attribute__((always_inline)) {
+    v = max ? wave_max(v) : wave_sum(v);
+    if (W > 1) {
+      if (lane == 0) red[k][slot][wave] = v;
+      __syncthreads();
+      v = red[k][slot][0];
+#pragma unroll
+      for (int i = 1; i < W; ++i) v = max ? fmaxf(v, red[k][slot][i]) : v + red[k][slot][i];
+    }
+    return v;
+  };
+  const uint16_t* xr = x + row * cols;
+  uint16_t* orow = out + row * cols;
+  u16x8 xv[NC], gv[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int j = (c * T + t) * 8;
+    xv[c] = gv[c] = (u16x8)(uint16_t)0;
+    const bool all = (c + 1) * T * 8 <= cols;  // uniform: no lane of the row needs a check
+    if (live && (all || j + 8 <= cols)) {
+      xv[c] = NT ? __builtin_nontemporal_load((const u16x8_any*)(xr + j)) : *(const u16x8_any*)(xr + j);
+      gv[c] = *(const u16x8_any*)(gain + j);
+    } else if (live && j < cols) {
+#pragma unroll
+      for (int e = 0; e < 7; ++e)
+        if (j + e < cols) {
+          xv[c][e] = xr[j + e];
+          gv[c][e] = gain[j + e];
+        }
+    }
   }
-  if (bad_local) g_bad = 1;
-  __syncthreads();
-  const bool gain_bad = g_bad != 0;
-  // The block's combine of the per-wave partials, in a fixed order so every wave gets the same
-  // value. A slot is rewritten only after the next barrier, which every reader has passed after
-  // its read.
-  auto block_sum = [&](int k, float v) {
-    if (lane == 0) red[k][w] = v;
-    __syncthreads();
-    float s = red[k][0];
+  float y[P];
+  float ss = 0.f;
+  bool bad = false;
 #pragma unroll
-    for (int i = 1; i < kSplit; ++i) s += red[k][i];
-    return s;
-  };
-  auto block_max = [&](int k, float v) {
-    if (lane == 0) red[k][w] = v;
-    __syncthreads();
-    float m = red[k][0];
+  for (int i = 0; i < P; ++i) {
+    y[i] = bits_f32((uint32_t)xv[i / 8][i % 8] << 16);
+    ss = __builtin_fmaf(y[i], y[i], ss);  // a bf16 square is exact in f32
+    bad |= !(__builtin_fabsf(bits_f32((uint32_t)gv[i / 8][i % 8] << 16)) < 0x1p120f);
+  }
+  ss = combine(0, bad ? INFINITY : ss, false);
+  const bool exact = !__builtin_isfinite(ss);  // uniform over the row's waves
+  const float ms = __fadd_rn(__fdiv_rn(ss, (float)cols), eps);  // fp_div, then clip Add eps
+  const float r = sqrt_rn(ms);                                    // FpUnaryOp::Sqrt
+  const float rinv = __fdiv_rn(1.0f, r);
+  float mx = -INFINITY;
 #pragma unroll
-    for (int i = 1; i < kSplit; ++i) m = fmaxf(m, red[k][i]);
-    return m;
-  };
-  const int e0 = ((w * CPW) * 64 + lane) * 8;  // first element of this lane's chunk 0; chunk c adds c * 512
-
-  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
-    const uint16_t* xr = x + row * cols;
-    i32x4_t v[CPW];
+  for (int c = 0; c < NC; ++c) {
+    const int past = cols - (c * T + t) * 8;  // elements of the chunk inside the row
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) v[c] = __builtin_nontemporal_load((const i32x4_t*)(xr + e0 + c * 512));
-    // Sum of squares by v_dot2_f32_bf16 on the packed pairs. The reference rounds each square and
-    // then each partial sum; the squares of bf16 values are exact in f32, and its reduction order
-    // is not this one anyway, so the sums agree to f32 rounding.
-    float ss = 0.f;
+    for (int i = 0; i < 8; i += 2) {
+      float* v = y + c * 8 + i;
 #pragma unroll
-    for (int c = 0; c < CPW; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ss = dot2_bf16(v[c][e], v[c][e], ss);
-    ss = block_sum(0, wave_sum(ss));
-    uint16_t* orow = out + row * cols;
-    if (!__builtin_isfinite(ss) || gain_bad) {  // block-uniform
-      if (w == 0) row_exact(orow, xr, gain, cols, eps, lane);
-      __syncthreads();  // every wave has read red[0] before the next row rewrites it
-      continue;
+      for (int e = 0; e < 2; ++e) v[e] = div_cr(v[e] * bits_f32((uint32_t)gv[c][i + e] << 16), r, rinv);
+      const uint32_t u = pack_bf16(v[0], v[1]);
+      v[0] = lo_raw(u);
+      v[1] = hi_raw(u);
     }
-    const float ms = __fadd_rn(__fdiv_rn(ss, cols_f), eps);  // fp_div, then clip Add eps
-    const float r = sqrt_rn(ms);                              // FpUnaryOp::Sqrt
-    const float rinv = __fdiv_rn(1.0f, r);
-    // y = bf16((x * g) / r), kept packed; row max on the f32 values
-    float mx = -INFINITY;
+    if ((c + 1) * T * 8 > cols) {  // uniform
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      f32x4_t g0 = *(const f32x4_t*)(sg + e0 + c * 512);
-      f32x4_t g1 = *(const f32x4_t*)(sg + e0 + c * 512 + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        uint32_t u = (uint32_t)v[c][e];
-        float glo = e < 2 ? g0[2 * e] : g1[2 * e - 4];
-        float ghi = e < 2 ? g0[2 * e + 1] : g1[2 * e - 3];
-        float ylo = div_cr(lo_raw(u) * glo, r, rinv);
-        float yhi = div_cr(hi_raw(u) * ghi, r, rinv);
-        mx = fmaxf(mx, fmaxf(ylo, yhi));
-        v[c][e] = (int)pack_bf16(ylo, yhi);
-      }
+      for (int i = 0; i < 8; ++i) y[c * 8 + i] = i < past ? y[c * 8 + i] : -INFINITY;
     }
-    mx = block_max(1, wave_max(mx));
-    mx = bits_f32(pack_bf16(mx, mx) << 16);  // the max of the committed bf16 values
-    // softmax: e = exp(y - max) kept in f32, s = sum(e), out = bf16(e / s)
-    const float L2E = 1.4426950408889634f;
-    const float mxl = mx * L2E;
-    float ex[CPW][8];
-    float s = 0.f;
 #pragma unroll
-    for (int c = 0; c < CPW; ++c)
+    for (int i = 0; i < 8; i += 2) mx = fmaxf(fmaxf(mx, y[c * 8 + i]), y[c * 8 + i + 1]);
+  }
+  mx = combine(1, mx, true);
+  const float L2E = 1.4426950408889634f;
+  const float mxl = mx * L2E;
+  float s = 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        uint32_t u = (uint32_t)v[c][e];
-        ex[c][2 * e] = __builtin_amdgcn_exp2f(__builtin_fmaf(lo_raw(u), L2E, -mxl));
-        ex[c][2 * e + 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(hi_raw(u), L2E, -mxl));
-        s += ex[c][2 * e];
-        s += ex[c][2 * e + 1];
-      }
-    s = block_sum(2, wave_sum(s));
-    const float sinv = __builtin_amdgcn_rcpf(s);
+  for (int i = 0; i < P; ++i) {
+    y[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[i], L2E, -mxl));
+    s += y[i];
+  }
+  s = combine(2, s, false);
+  if (!live) return;
+  if (exact) {
+    if (wave == 0) row_exact(orow, xr, gain, cols, eps, lane);
+    return;
+  }
+  const float sinv = __builtin_amdgcn_rcpf(s);
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      i32x4_t o;
+  for (int c = 0; c < NC; ++c) {
+    const int j = (c * T + t) * 8;
+    uint32_t w[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = (int)pack_bf16(ex[c][2 * e] * sinv, ex[c][2 * e + 1] * sinv);
-      __builtin_nontemporal_store(o, (i32x4_t*)(orow + e0 + c * 512));
+    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(y[c * 8 + 2 * e] * sinv, y[c * 8 + 2 * e + 1] * sinv);
+    const u16x8 o = __builtin_bit_cast(u16x8, w);
+    const bool all = (c + 1) * T * 8 <= cols;
+    if (all || j + 8 <= cols) {
+      if (NT)
+        __builtin_nontemporal_store(o, (u16x8_any*)(orow + j));
+      else
+        *(u16x8_any*)(orow + j) = o;
+    } else if (j < cols) {
+#pragma unroll
+      for (int e = 0; e < 7; ++e)
+        if (j + e < cols) orow[j + e] = o[e];
     }
   }
 }
 
-template <int CPW>
-void rs_split_launch(hipStream_t s, uint16_t* out, const uint16_t* x, const uint16_t* g, int64_t rows, float eps) {
-  static int64_t resident_blocks = [] {
-    int dev = 0, per_cu = 1, cus = 1;
-    (void)hipGetDevice(&dev);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_rmsnorm_softmax_split<CPW>, 64 * kSplit, 0) !=
-            hipSuccess ||
-        per_cu < 1)
-      per_cu = 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
-    return (int64_t)per_cu * cus;
-  }();
-  int64_t blocks = rows < resident_blocks ? rows : resident_blocks;
-  hipLaunchKernelGGL(k_rmsnorm_softmax_split<CPW>, dim3((unsigned)blocks), dim3(64 * kSplit), 0, s, out, x, g, rows,
-                     (float)(kSplit * CPW * 512), eps);
+template <int P, int W>
+void rs_row_launch(hipStream_t s, uint16_t* out, const uint16_t* x, const uint16_t* g, int64_t rows, int64_t cols,
+                   float eps, bool stream) {
+  constexpr int R = W < 4 ? 4 / W : 1;
+  const dim3 grid((unsigned)((rows + R - 1) / R)), block(W < 4 ? 256 : 64 * W);
+  if (stream)
+    hipLaunchKernelGGL((k_rmsnorm_softmax_row<P, W, true>), grid, block, 0, s, out, x, g, rows, (int)cols, eps);
+  else
+    hipLaunchKernelGGL((k_rmsnorm_softmax_row<P, W, false>), grid, block, 0, s, out, x, g, rows, (int)cols, eps);
 }
 
-// Any column count: the exact per-element path, one wave per row.
+// Rows past 32768 columns: the exact per-element path, one wave per row.
 __global__ void __launch_bounds__(256) k_rmsnorm_softmax_any(uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
                                                              const uint16_t* __restrict__ gain, int64_t rows, int64_t cols,
                                                              float eps) {
@@ -429,18 +428,40 @@ void launch_rmsnorm_softmax(hipStream_t s, uint16_t* out, const uint16_t* x, con
                             int64_t cols, float eps) {
   require((rows + 3) / 4 < (1ll << 31), "rmsnorm_softmax: too many rows");
   require(cols < (1ll << 30), "rmsnorm_softmax: too many columns");
-  bool aligned = ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0) && ((uintptr_t)gain % 16 == 0);
-  if (aligned && cols % 512 == 0 && cols <= 8192) {
-    switch (cols / 512) {
-      case 1: rs_dma_launch<1>(s, out, x, gain, rows, eps); break;
-      case 2: rs_dma_launch<2>(s, out, x, gain, rows, eps); break;
-      case 4: rs_dma_launch<4>(s, out, x, gain, rows, eps); break;
-      case 8: rs_dma_launch<8>(s, out, x, gain, rows, eps); break;
-      case 16: rs_split_launch<4>(s, out, x, gain, rows, eps); break;
-      default:
-        hipLaunchKernelGGL(k_rmsnorm_softmax_any, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, out, x, gain, rows,
-                           cols, eps);
-    }
+  // Measured as the kernel alone in a recorded graph, us (one box; DMA is k_rmsnorm_softmax_dma, exact
+  // the per-element path that took every column count the DMA form does not):
+  //     rows, cols     row kernel   before        rows, cols     row kernel   before
+  //     500, 512          3.1     4.4 (DMA)       500, 3072         4.5     41 (exact)
+  //     32768, 1024      24.4    26.2 (DMA)       8192, 4096       26.8     25.7 (DMA)
+  //     500, 4096         4.5    12.2 (DMA)       4096, 8192       28.7     30.8 (rows split over 4 waves)
+  // so the DMA form is kept where it is the faster one, past 6144 rows of 4096 (15.3 against 16.0 at 4096
+  // rows). W and P are the best of one to sixteen waves a row; wider rows want more waves while the
+  // result is small (2048 columns: 3.7 us with 4 waves against 3.9 with 2 at 500 rows; 32.4 against 26.2 at
+  // 16384). Past 10 MiB a tensor the accesses stream past the caches (1500, 4096: 7.9 against 9.1 us;
+  // at 4 MiB 5.3 against 4.5).
+  const bool aligned = (((uintptr_t)x | (uintptr_t)out | (uintptr_t)gain) & 15) == 0;
+  const bool stream = rows * cols * 2 >= (10ll << 20);
+  if (aligned && cols == 4096 && rows >= 6144) {
+    rs_dma_launch<8>(s, out, x, gain, rows, eps);
+  } else if (cols <= 32768 && rows < (1ll << 31)) {
+    if (cols <= 512)
+      rs_row_launch<8, 1>(s, out, x, gain, rows, cols, eps, stream);
+    else if (cols <= 1024)
+      rs_row_launch<16, 1>(s, out, x, gain, rows, cols, eps, stream);
+    else if (cols <= 2048 && !stream)
+      rs_row_launch<8, 4>(s, out, x, gain, rows, cols, eps, stream);
+    else if (cols <= 2048)
+      rs_row_launch<16, 2>(s, out, x, gain, rows, cols, eps, stream);
+    else if (cols <= 3072 && stream)
+      rs_row_launch<24, 2>(s, out, x, gain, rows, cols, eps, stream);
+    else if (cols <= 4096)
+      rs_row_launch<16, 4>(s, out, x, gain, rows, cols, eps, stream);
+    else if (cols <= 8192)
+      rs_row_launch<16, 8>(s, out, x, gain, rows, cols, eps, stream);
+    else if (cols <= 16384)
+      rs_row_launch<16, 16>(s, out, x, gain, rows, cols, eps, stream);
+    else
+      rs_row_launch<32, 16>(s, out, x, gain, rows, cols, eps, stream);
   } else {
     hipLaunchKernelGGL(k_rmsnorm_softmax_any, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, out, x, gain, rows,
                        cols, eps);

@@ -1,0 +1,54 @@
+"""RMSNorm -> softmax over any row length (k_rmsnorm_softmax_row): each choice of waves per row at the
+first, last and ragged columns of its range, rows that start at odd addresses, and the streamed form."""
+import numpy as np
+import pytest
+
+import furiosa_hip as fh  # noqa: F401  (the library under test)
+from oracle import emulator as emu
+from test_gpu_fused import bf16, close_chain, rmsnorm_bound, rmsnorm_softmax_numpy
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(3, 1), (5, 7), (9, 8), (6, 63), (5, 511), (5, 513), (7, 1001), (3, 1024), (5, 1025), (3, 2047), (2, 2049),
+          (3, 4095), (2, 4097), (3, 8191), (2, 8193), (2, 16383), (1, 16385), (2, 32767), (1, 32768), (1, 32769),
+          # past 10 MiB a tensor: streamed accesses, two waves a row up to 3072 columns
+          (5200, 1025), (3000, 2047), (2601, 2049), (1710, 3072), (1706, 3073), (6144, 4096)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_rmsnorm_softmax_rows(rt, shape):
+    rows, cols = shape
+    rng = np.random.default_rng(rows + cols)
+    x, g = bf16(rng, rows * cols), bf16(rng, cols, 0.1, 1.0)
+    want = rmsnorm_softmax_numpy(x, g, rows, cols, 1e-6)
+    out = rt.upload(np.full(rows * cols + 8, 0x5A5A, np.uint16))
+    print(f"rmsnorm_softmax rows {rows}x{cols}", flush=True)
+    rt.rmsnorm_softmax(out, rt.upload(x), rt.upload(g), rows, cols, 1e-6)
+    got = out.read(np.uint16)
+    assert np.all(got[rows * cols:] == 0x5A5A)  # nothing past the last row
+    close_chain(emu.bf16_to_f32(got[:rows * cols]).reshape(rows, cols), want, hard=rmsnorm_bound(x, g, rows, cols, 1e-6),
+                frac_beyond=1e-4)
+
+
+@pytest.mark.parametrize("cols", [65, 1000, 3001, 5000])
+def test_rmsnorm_softmax_rows_nonfinite(rt, cols):
+    """A NaN, an infinity and a square past f32's range each send their own row, and no other, through
+    the reference's per-element rules; so does a gain of 2^121 every row."""
+    rows = 9
+    rng = np.random.default_rng(cols)
+    x = bf16(rng, rows * cols).reshape(rows, cols)
+    x[1, 0], x[3, cols - 1], x[6, 33] = emu.f32_to_bf16(np.array([np.nan, np.inf, 1e20], np.float32))
+    for huge in (False, True):
+        g = bf16(rng, cols, 0.1, 1.0)
+        if huge:
+            g[cols - 2] = emu.f32_to_bf16(np.array([2.0 ** 121], np.float32))[0]
+        want = emu.bf16_to_f32(emu.rmsnorm_softmax(x.ravel(), g, rows, cols, 1e-6)).reshape(rows, cols)
+        out = rt.alloc(rows * cols * 2)
+        rt.rmsnorm_softmax(out, rt.upload(x.ravel()), rt.upload(g), rows, cols, 1e-6)
+        got = emu.bf16_to_f32(out.read(np.uint16)).reshape(rows, cols)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        fin = ~np.isnan(want)
+        assert fin[[0, 2, 4, 5, 7, 8]].all() and np.isnan(want[[1, 3]]).all()
+        if not huge:
+            bound = rmsnorm_bound(x.ravel(), g, rows, cols, 1e-6)
+            close_chain(got[fin], want[fin], frac_beyond=1e-4, hard=bound[fin])
