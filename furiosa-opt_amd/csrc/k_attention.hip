@@ -116,9 +116,8 @@ struct AttnCfg {
 __device__ __forceinline__ int vt_pos(int kk) { return (kk & ~15) + ((kk & 4) << 1) + ((kk & 8) >> 1) + (kk & 3); }
 
 // S^T tile pair for the 64 keys of one K buffer: keys kt*32 + 8*(r/4) + 4g + r%4 of s[kt][r].
-template <int D>
-__device__ __forceinline__ void qk(const uint8_t* __restrict__ sK, const i32x4_t (&qf)[AttnCfg<D>::KS],
-                                   f32x16_t (&s)[2], int g, int col) {
+template <int D, typename Q>
+__device__ __forceinline__ void qk(const uint8_t* __restrict__ sK, const Q& qf, f32x16_t (&s)[2], int g, int col) {
   using C = AttnCfg<D>;
 #pragma unroll
   for (int kt = 0; kt < 2; ++kt) {
@@ -133,14 +132,15 @@ __device__ __forceinline__ void qk(const uint8_t* __restrict__ sK, const i32x4_t
 }
 
 // One step: S of the block (K from sK), its softmax, then its PV product (V^T from sVt).
-template <int D, bool MASK, bool GIVEN>
+// qf[ks] is the wave's Q fragment of k-step ks (registers, or read from LDS).
+template <int D, bool MASK, bool GIVEN, typename Q>
 __device__ __forceinline__ void attn_step(const uint8_t* __restrict__ sK, const uint8_t* __restrict__ sVt,
-                                          const i32x4_t (&qf)[AttnCfg<D>::KS], f32x16_t (&o)[AttnCfg<D>::DT],
+                                          const Q& qf, f32x16_t (&o)[AttnCfg<D>::DT],
                                           float& m_run, float& l_part,
                                           int kv0, int lim, float inv_sd, int g, int col) {
   using C = AttnCfg<D>;
   f32x16_t sc[2];
-  qk<D>(sK, qf, sc, g, col);
+  qk<D, Q>(sK, qf, sc, g, col);
   // Scaled sums first, then the block max over them (the max of products is the product of the
   // max, and bf16 rounding is monotonic, so the max commutes with both). Taking it on product
   // results also spares the quieting of each operand that a max of raw MFMA outputs needs.
@@ -227,6 +227,16 @@ __device__ __forceinline__ void attn_step(const uint8_t* __restrict__ sK, const 
       o[t] = mma(vf, pf[c], o[t]);
     }
   }
+}
+
+// bf16(bf16(o) / denom) of two elements, packed: correctly rounded quotients (rinv = RN(1 / denom)); an
+// infinite o (an infinite value in V) divides to itself, where div_cr's remainder would be NaN.
+__device__ __forceinline__ uint32_t normalized_pair(float o0, float o1, float denom, float rinv) {
+  const uint32_t ob = pack_bf16(o0, o1);
+  const float a = __builtin_bit_cast(float, ob << 16), b = __builtin_bit_cast(float, ob & 0xffff0000u);
+  const float qa = __builtin_isinf(a) ? a : div_cr(a, denom, rinv);
+  const float qb = __builtin_isinf(b) ? b : div_cr(b, denom, rinv);
+  return pack_bf16(qa, qb);
 }
 
 template <int D, bool GIVEN>
@@ -399,16 +409,221 @@ __global__ void __launch_bounds__(kNT, 2 * 4 / kWaves) k_attn_fwd(uint16_t* __re
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const int blk = bp + d;
-          const uint32_t ob = pack_bf16(o[t][blk * 4 + 2 * e], o[t][blk * 4 + 2 * e + 1]);
-          const float a = __builtin_bit_cast(float, ob << 16), b = __builtin_bit_cast(float, ob & 0xffff0000u);
-          // An infinite o (an infinite value in V) divides to itself; div_cr's remainder would be NaN.
-          const float qa = __builtin_isinf(a) ? a : div_cr(a, denom, rinv);
-          const float qb = __builtin_isinf(b) ? b : div_cr(b, denom, rinv);
-          wv[d][e] = (int)pack_bf16(qa, qb);
+          wv[d][e] = (int)normalized_pair(o[t][blk * 4 + 2 * e], o[t][blk * 4 + 2 * e + 1], denom, rinv);
         }
       const i32x4_t q4 = regroup8(wv[0], wv[1]);
       if (myq < seq) *(i32x4_t*)(orow + t * 32 + 8 * bp + 8 * g) = q4;
     }
+}
+
+// ---- few query blocks: the keys of a step split over wave groups -----------------------------------
+//
+// With few heads or short sequences the 256-query workgroups above leave most CUs idle while each
+// walks its keys one 64-key block at a time. Here a workgroup of eight waves is QG groups of 32 queries
+// by KG groups of keys: a step stages KG blocks of 64 keys, wave (qg, kg) folds block kg into its own
+// (max, sum, O), and the KG partial results of a query group are combined at the end through LDS with
+// the online softmax's rescale, one 32-row tile of O per wave. Bound by latency: a step of the 2 x 4 form
+// takes 3.4 us (loads, LDS stores, barrier, S, softmax and PV in turn: the four blocks fill the LDS, so
+// nothing is double-buffered), of the 4 x 2 form 2.3 us, against 1.8 us for one block of the 256-query form.
+// Four waves of one query group by four key groups measured no faster (600 keys: 15.4 us). The running max starts at a finite
+// value below any logit (kLow), so a wave that has seen no visible key yet holds (kLow, 0, 0) and
+// weighs nothing in the combine.
+constexpr float kLow = -2.3e38f;  // kLow * log2(e) is still finite
+
+template <int D, int QG, int KG>
+struct SplitCfg {
+  using C = AttnCfg<D>;
+  static constexpr int NW = QG * KG, NT = 64 * NW;  // waves, threads
+  static constexpr int NBUF = KG > 2 ? 1 : 2;  // LDS holds four blocks
+  static constexpr int KL = KG * kBN * C::CH / NT;            // K chunks per thread and step
+  static constexpr int VG = KG * kBN / 4 * C::CH;              // (4-key group, chunk) pairs per step
+  static constexpr int VL = (VG + NT - 1) / NT;
+  static constexpr int STAGES = NBUF * KG * C::STAGE;
+  static constexpr int SUMS = NW * 64 * (C::DT * 16 + 2) * 4;  // the partial results, after the loop
+  // Eight waves at D = 128 with a step's next 256 keys in registers have none left for Q: its fragments
+  // are read from LDS each step (24 registers spilled otherwise).
+  static constexpr bool QLDS = D == 128 && KG == 4 && NW == 8;
+  static constexpr int LDS = (STAGES > SUMS ? STAGES : SUMS) + (QLDS ? QG * 32 * C::KROW : 0);
+  static_assert(LDS <= 160 * 1024, "");
+};
+
+template <int D, int QG, int KG>
+__global__ void __launch_bounds__(64 * QG * KG, QG * KG <= 4 ? 1 : 2) k_attn_split(uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
+                                                       const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                                       int32_t heads_total, int32_t seq, int32_t nqb, float inv_sd,
+                                                       int32_t causal) {
+  using C = AttnCfg<D>;
+  using S = SplitCfg<D, QG, KG>;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int bid = blockIdx.x;
+  const int qb = nqb - 1 - bid / heads_total;  // heaviest query blocks first
+  const int64_t head = bid % heads_total;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qg = wave % QG, kg = wave / QG;
+  const int g = lane >> 5, col = lane & 31;
+  const int q0 = qb * 32 * QG, q0w = q0 + qg * 32, myq = q0w + col;
+  const int lim = causal ? min(myq, seq - 1) : seq - 1;
+
+  const uint32_t head_bytes = (uint32_t)seq * D * 2;
+  const int64_t at = head * (int64_t)seq * D;
+  const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)(q + at), (short)0, (int)head_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)(k + at), (short)0, (int)head_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)(v + at), (short)0, (int)head_bytes, 0x00020000);
+
+  // Thread's chunks: K row RPI i + tid / CH of the step, column tid % CH; V keys 4 (tid % 16) .. + 3 of
+  // block BPI i + tid / (16 CH), column tid / 16 % CH. One per-lane address each for loads and stores,
+  // the rest constant.
+  constexpr int RPI = S::NT / C::CH, BPI = S::NT / (16 * C::CH);
+  static_assert(kBN % RPI == 0 && (BPI > 0 || S::VL == 1), "");
+  const int vblk = tid / (16 * C::CH), vcc = tid / 16 % C::CH, vkq = tid % 16;
+  const uint32_t koff = (uint32_t)((tid / C::CH * D + tid % C::CH * 8) * 2);
+  const uint32_t voff = (uint32_t)(((vblk * kBN + vkq * 4) * D + vcc * 8) * 2);
+  const int kst = tid / C::CH * C::KROW + tid % C::CH * 16;
+  const int vst = vblk * C::STAGE + C::KBYTES + vcc * 8 * C::VROW + vt_pos(vkq * 4) * 2;
+  const bool has_v = S::VG % S::NT == 0 || tid < S::VG;
+  i32x4_t kreg[S::KL];
+  i32x4_t vreg[S::VL][4];
+  auto load = [&](int kv0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < S::KL; ++i) kreg[i] = __builtin_amdgcn_raw_buffer_load_b128(rk, koff, (kv0 + i * RPI) * D * 2, 0);
+    if (has_v)
+#pragma unroll
+      for (int i = 0; i < S::VL; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          vreg[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rv, voff + j * D * 2, (kv0 + i * BPI * kBN) * D * 2, 0);
+  };
+  auto store = [&](int buf) __attribute__((always_inline)) {
+    uint8_t* base = lds + buf * KG * C::STAGE;
+#pragma unroll
+    for (int i = 0; i < S::KL; ++i)
+      *(i32x4_t*)(base + kst + i * RPI / kBN * C::STAGE + i * RPI % kBN * C::KROW) = kreg[i];
+    if (has_v)
+#pragma unroll
+      for (int i = 0; i < S::VL; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {  // column 8 vcc + e: four keys, as two packed pairs
+          const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+          const uint32_t w0 = __builtin_amdgcn_perm((uint32_t)vreg[i][1][e >> 1], (uint32_t)vreg[i][0][e >> 1], sel);
+          const uint32_t w1 = __builtin_amdgcn_perm((uint32_t)vreg[i][3][e >> 1], (uint32_t)vreg[i][2][e >> 1], sel);
+          *(i32x2_t*)(base + vst + i * BPI * C::STAGE + e * C::VROW) = i32x2_t{(int)w0, (int)w1};
+        }
+  };
+
+  i32x4_t qf[C::KS];
+#pragma unroll
+  for (int ks = 0; ks < C::KS; ++ks)
+    qf[ks] = __builtin_amdgcn_raw_buffer_load_b128(rq, (uint32_t)(myq * D + g * 8) * 2, ks * 32, 0);
+  load(0);
+  uint8_t* sQ = lds + S::NBUF * KG * C::STAGE + (qg * 32 + col) * C::KROW + g * 16;
+  if (S::QLDS && kg == 0)  // read after the first step's barrier
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) *(i32x4_t*)(sQ + ks * 32) = qf[ks];
+  struct QFromLds {
+    const uint8_t* p;
+    __device__ __forceinline__ i32x4_t operator[](int ks) const { return *(const i32x4_t*)(p + ks * 32); }
+  };
+  f32x16_t o[C::DT];
+#pragma unroll
+  for (int t = 0; t < C::DT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+  float m_run = kLow, l_part = 0.f;
+
+  const int kv_end = causal ? min(seq, q0 + 32 * QG) : seq;
+  const int nstep = (kv_end + KG * kBN - 1) / (KG * kBN);
+  const int vis = causal ? min(q0w, seq - 1) : seq - 1;  // last key every query of the wave sees
+  for (int j = 0; j < nstep; ++j) {
+    const int buf = S::NBUF == 1 ? 0 : j & 1;
+    store(buf);
+    __syncthreads();
+    if (j + 1 < nstep) load((j + 1) * KG * kBN);
+    __builtin_amdgcn_sched_barrier(0);
+    const int kv0 = (j * KG + kg) * kBN;
+    const uint8_t* sK = lds + (buf * KG + kg) * C::STAGE;
+    auto block = [&](const auto& q) __attribute__((always_inline)) {
+      if (kv0 + kBN - 1 <= vis)  // wave-uniform
+        attn_step<D, false, false>(sK, sK + C::KBYTES, q, o, m_run, l_part, kv0, lim, inv_sd, g, col);
+      else if (kv0 < kv_end && !(causal && kv0 > q0w + 31))  // wave-uniform
+        attn_step<D, true, false>(sK, sK + C::KBYTES, q, o, m_run, l_part, kv0, lim, inv_sd, g, col);
+    };
+    if constexpr (S::QLDS)
+      block(QFromLds{sQ});
+    else
+      block(qf);
+    if (S::NBUF == 1) __syncthreads();  // two buffers: the next store's was last read a step ago
+  }
+  if (S::NBUF > 1) __syncthreads();
+
+  // Combine. Wave (qg, kg) finishes O tiles kg, kg + KG, ..; the others' tiles and every wave's max and
+  // sum go through LDS (a lane's values 256 bytes apart: no bank conflicts).
+  float* so = (float*)lds;
+  float* sml = so + S::NW * C::DT * 16 * 64;
+#pragma unroll
+  for (int t = 0; t < C::DT; ++t)
+    if (t % KG != kg)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) so[((wave * C::DT + t) * 16 + r) * 64 + lane] = o[t][r];
+  {
+    const LanePair lp = half_pair(l_part);  // the query's other keys live in lane ^ 32
+    l_part = lp.lo + lp.hi;
+  }
+  sml[(wave * 2 + 0) * 64 + lane] = m_run;
+  sml[(wave * 2 + 1) * 64 + lane] = l_part;
+  __syncthreads();
+  float m = kLow, f[KG], l = 0.f;
+#pragma unroll
+  for (int i = 0; i < KG; ++i) m = __builtin_fmaxf(m, sml[((i * QG + qg) * 2) * 64 + lane]);
+#pragma unroll
+  for (int i = 0; i < KG; ++i) {
+    f[i] = __builtin_amdgcn_exp2f((sml[((i * QG + qg) * 2) * 64 + lane] - m) * kL2E);
+    l += f[i] * sml[((i * QG + qg) * 2 + 1) * 64 + lane];
+  }
+  const float denom = l + kEps;
+  const float rinv = __fdiv_rn(1.0f, denom);
+  uint16_t* orow = out + at + (int64_t)myq * D;
+#pragma unroll
+  for (int t = 0; t < C::DT; ++t) {
+    if (t % KG != kg) continue;  // wave-uniform
+    float s[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+    for (int i = 0; i < KG; ++i) {
+      const int w = i * QG + qg;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float ov = w == wave ? o[t][r] : so[((w * C::DT + t) * 16 + r) * 64 + lane];
+        s[r] = __builtin_fmaf(f[i], ov, s[r]);
+      }
+    }
+    // out[myq][d] = bf16(bf16(o) / (l + EPS)), stored as in k_attn_fwd
+#pragma unroll
+    for (int bp = 0; bp < 4; bp += 2) {
+      i32x2_t wv[2];
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) wv[d][e] = (int)normalized_pair(s[(bp + d) * 4 + 2 * e], s[(bp + d) * 4 + 2 * e + 1], denom, rinv);
+      const i32x4_t q4 = regroup8(wv[0], wv[1]);
+      if (myq < seq) *(i32x4_t*)(orow + t * 32 + 8 * bp + 8 * g) = q4;
+    }
+  }
+}
+
+template <int D, int QG, int KG>
+void launch_split(hipStream_t s, uint16_t* out, const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t ht,
+                  int64_t seq, float inv_sd, int causal) {
+  constexpr int lds = SplitCfg<D, QG, KG>::LDS;
+  static bool attr_set = false;
+  if (!attr_set) {
+    FO_HIP(hipFuncSetAttribute((const void*)k_attn_split<D, QG, KG>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    attr_set = true;
+  }
+  const int64_t nqb = (seq + 32 * QG - 1) / (32 * QG);
+  hipLaunchKernelGGL((k_attn_split<D, QG, KG>), dim3((unsigned)(ht * nqb)), dim3(64 * QG * KG), lds, s, out, q, k, v, (int32_t)ht,
+                     (int32_t)seq, (int32_t)nqb, inv_sd, causal);
 }
 
 template <int D, bool GIVEN>
@@ -435,7 +650,27 @@ void launch_attention_prefill(hipStream_t s, uint16_t* out, const uint16_t* q, c
   require(ht * nqb < (1ll << 31) && (seq + 2 * kBN) * head_dim * 2 < (1ll << 31), "attention: shape too large");
   dim3 grid((unsigned)(ht * nqb));
   const float inv_sd = 1.0f / sqrt_d;
-  if (head_dim == 128)
+  // Which form, by the workgroups each would have (WG64 and WG128: a workgroup per 64 or 128 queries of a
+  // head). Kernel alone in a recorded graph, D = 128 causal, us (one box):
+  //     heads, seq    WG64   2 x 4 groups    WG128   4 x 2 groups    256 queries
+  //     1, 600          10       14.1            5       16.3            22.4
+  //     16, 600        160       15.5           80       17.3            23.2
+  //     16, 1024       256       21.0          128       24.9            34.5
+  //     64, 300        320       16.8          192       13.1            16.3
+  //     64, 600        640       31.6          320       21.4            26.6
+  //     32, 2048      1024       87            512       60.4            66.3
+  //     128, 512      1024       43            512       27.4            25.0
+  //     64, 2048      2048      174           1024      120             106.5
+  //     16, 64          16        7.4           16        7.0             7.1
+  // and D = 64 alike (16, 600: 10.3, 11.4, 17.1). A given row maximum keeps the 256-query form.
+  const int64_t wg64 = ht * ((seq + 63) / 64), wg128 = ht * ((seq + 127) / 128);
+  if (!row_max && wg64 <= 256 && seq > 64) {
+    head_dim == 128 ? launch_split<128, 2, 4>(s, out, q, k, v, ht, seq, inv_sd, causal)
+                    : launch_split<64, 2, 4>(s, out, q, k, v, ht, seq, inv_sd, causal);
+  } else if (!row_max && (wg128 <= 320 || (wg128 <= 512 && seq >= 1024))) {
+    head_dim == 128 ? launch_split<128, 4, 2>(s, out, q, k, v, ht, seq, inv_sd, causal)
+                    : launch_split<64, 4, 2>(s, out, q, k, v, ht, seq, inv_sd, causal);
+  } else if (head_dim == 128)
     row_max ? launch_d<128, true>(s, grid, out, q, k, v, row_max, ht, seq, nqb, inv_sd, causal)
             : launch_d<128, false>(s, grid, out, q, k, v, row_max, ht, seq, nqb, inv_sd, causal);
   else

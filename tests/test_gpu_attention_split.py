@@ -1,0 +1,57 @@
+"""Attention with a step's keys split over wave groups (k_attn_split): both forms and the 256-query form on
+either side of their rule, at the edges of query groups, key blocks and steps."""
+import numpy as np
+import pytest
+
+from oracle import emulator as emu
+from test_gpu_fused import attention_numpy, bf16, close_chain
+
+pytestmark = pytest.mark.gpu
+
+# (heads, seq): the 4 x 2 form up to 64 keys, the 2 x 4 form over several steps of 256 keys, then the 4 x 2 form (more
+# than 256 workgroups of 64 queries, at most 320 of 128), then just past it.
+CASES = [(1, 1), (3, 31), (2, 32), (5, 33), (2, 63), (2, 64), (3, 65), (2, 129), (1, 255), (2, 256), (1, 257), (2, 511),
+         (1, 513), (1, 800), (257, 40), (100, 150), (64, 257), (52, 513), (36, 1025), (330, 90)]
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_attention_split(rt, case, d, causal):
+    h, s = case
+    sqrt_d = np.float32(8.0 if d == 64 else 11.313708)
+    rng = np.random.default_rng(h * 10007 + s)
+    q, k, v = (bf16(rng, h * s * d) for _ in range(3))
+    out = rt.upload(np.full(h * s * d + 8, 0x5A5A, np.uint16))
+    print(f"attention split {h}x{s}x{d} causal={causal}", flush=True)
+    rt.attention_prefill(out, rt.upload(q), rt.upload(k), rt.upload(v), 1, h, s, d, float(sqrt_d), causal)
+    raw = out.read(np.uint16)
+    assert np.all(raw[h * s * d:] == 0x5A5A)  # nothing past the last query
+    got = emu.bf16_to_f32(raw[:h * s * d]).reshape(h, s, d)
+    heads = range(h) if h <= 5 else sorted(set(int(x) for x in np.linspace(0, h - 1, 5)))
+    for i in heads:
+        sl = slice(i * s * d, (i + 1) * s * d)
+        ref, bound = attention_numpy(q[sl], k[sl], v[sl], s, d, sqrt_d, causal)
+        close_chain(got[i], ref, frac_beyond=2e-3, hard=bound)
+
+
+def test_attention_split_growing_logits(rt):
+    """Keys whose logits grow along the sequence, so every later block raises the running max by far
+    more than the rescale margin, and queries that see only the first, small ones."""
+    h, s, d = 2, 600, 128
+    rng = np.random.default_rng(9)
+    q = np.abs(rng.standard_normal((h, s, d))).astype(np.float32)
+    k = (rng.standard_normal((h, s, d)) * 0.1 + np.linspace(0.0, 3.0, s)[None, :, None]).astype(np.float32)
+    q, k = emu.f32_to_bf16(q.ravel()), emu.f32_to_bf16(k.ravel())
+    v = bf16(rng, h * s * d)
+    out = rt.alloc(h * s * d * 2)
+    rt.attention_prefill(out, rt.upload(q), rt.upload(k), rt.upload(v), 1, h, s, d, 11.313708, True)
+    got = emu.bf16_to_f32(out.read(np.uint16)).reshape(h, s, d)
+    # a causal row's own max: the chain over its visible keys alone (p rounds at that scale here)
+    for i in range(h):
+        sl = slice(i * s * d, (i + 1) * s * d)
+        for row in (0, 40, 64, 255, 256, 400, 599):
+            n = row + 1
+            qs, ks, vs = (t[sl].reshape(s, d)[:n].ravel() for t in (q, k, v))
+            ref, bound = attention_numpy(qs, ks, vs, n, d, np.float32(11.313708), False)
+            close_chain(got[i, row], ref[row], frac_beyond=2e-2, hard=bound[row])
