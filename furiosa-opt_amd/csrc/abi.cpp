@@ -2235,6 +2235,7 @@ void contraction_impl(fo_runtime* rt, fo_buffer* out, const fo_buffer* lhs, cons
             launch_gemm(rt->stream, O, L, R, ct, co, d, rt->gemm_ws);
             return;
           }
+          if (amax < lhs_len && bmax < rhs_len && launch_gemm_any(rt->stream, O, L, R, ct, co, d, rt->gemm_ws)) return;
         }
         // The wheel-decoded kernel: rows, columns and batch cells over any number of wheels
         // (live digits only; dead out cells zeroed first), when a 32 x 32 tile is at least a

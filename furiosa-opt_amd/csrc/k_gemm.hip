@@ -37,6 +37,7 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4_t;
+typedef i32x4_t i32x4_any_t __attribute__((aligned(1)));  // at any address
 typedef __attribute__((__vector_size__(16 * sizeof(int)))) int i32x16_t;
 typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2_t;
 typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8_t;
@@ -48,6 +49,8 @@ constexpr int kSwzShift = kRB == 64 ? 2 : 1;    // rows sharing a bank-group off
 
 // s_waitcnt immediate (gfx9 encoding): vector memory count <= n, LDS/scalar count 0, export any.
 constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | (7 << 4) | ((n >> 4) << 14); }
+
+constexpr int waitcnt_lgkm0 = 15 | (7 << 4) | (3 << 14);  // LDS / scalar count 0, vector memory left alone
 
 // Operand kinds. Per MFMA, each lane supplies FRAG bytes of k (16 for bf16 / i8, 32 for the
 // 8-bit floats: k = 64 per instruction); KSTEP = 2 * FRAG bytes of k per row per MFMA.
@@ -238,7 +241,10 @@ __device__ __forceinline__ bool combine_splits(const GemmArgs& g, int tile, int 
   return true;
 }
 
-template <int KIND, int OUT, int BM, int BN, int WM, int WN, int NS>
+// DMA: operand rows start at 16-byte addresses and K is whole 16-byte chunks. Otherwise (any element
+// alignment) the same tiles are staged through registers: unaligned 16-byte loads of stage s + 1 while
+// stage s is computed, the chunk that straddles the end of K element by element, then LDS writes.
+template <int KIND, int OUT, int BM, int BN, int WM, int WN, int NS, bool DMA>
 __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   using M = MfmaT<KIND>;
   using acc_t = typename M::acc_t;
@@ -413,6 +419,82 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
     }
   };
 
+  if constexpr (!DMA) {
+    using elem_t = std::conditional_t<EB == 2, uint16_t, uint8_t>;
+    // PF stages in registers ahead of the two in LDS (333, 1000, 777 bf16: 11.6 us with one, 9.1 with two,
+    // 9.5 with four). Rows past the operand's read its last row (their
+    // results are not stored).
+    constexpr int PF = 2;
+    i32x4_t ca[PF][A_CH], cb[PF][B_CH];
+    const uint8_t *pa[A_CH], *pb[B_CH];
+#pragma unroll
+    for (int i = 0; i < A_CH; ++i) {
+      const int64_t r = min((int64_t)(kRPC * (wave * A_CH + i) + lane / kCPR), rows_a - 1);
+      pa[i] = Abase + r * g.lda * EB + a_kc[i];
+    }
+#pragma unroll
+    for (int i = 0; i < B_CH; ++i) {
+      const int64_t r = min((int64_t)(kRPC * (wave * B_CH + i) + lane / kCPR), rows_b - 1);
+      pb[i] = Bbase + r * g.ldb * EB + b_kc[i];
+    }
+    auto part = [&](const uint8_t* p, uint32_t kc, uint32_t kb) __attribute__((always_inline)) {  // K's last stage
+      const uint32_t at = kb + kc;
+      if (at + 16 <= KB) return *(const i32x4_any_t*)(p + kb) + 0;
+      elem_t e[16 / EB];
+#pragma unroll
+      for (int i = 0; i < 16 / EB; ++i) e[i] = at + i * EB < KB ? ((const elem_t*)(p + kb))[i] : (elem_t)0;
+      return __builtin_bit_cast(i32x4_t, e);
+    };
+    auto load_stage = [&](int st, int u) __attribute__((always_inline)) {
+      const uint32_t kb = (uint32_t)(st0 + st) * kRB;
+      if (kb + kRB <= KB) {  // uniform
+#pragma unroll
+        for (int i = 0; i < A_CH; ++i) ca[u][i] = *(const i32x4_any_t*)(pa[i] + kb);
+#pragma unroll
+        for (int i = 0; i < B_CH; ++i) cb[u][i] = *(const i32x4_any_t*)(pb[i] + kb);
+      } else {
+#pragma unroll
+        for (int i = 0; i < A_CH; ++i) ca[u][i] = part(pa[i], a_kc[i], kb);
+#pragma unroll
+        for (int i = 0; i < B_CH; ++i) cb[u][i] = part(pb[i], b_kc[i], kb);
+      }
+    };
+    auto store_stage = [&](int buf, int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < A_CH; ++i) *(i32x4_t*)(sA(buf) + (wave * A_CH + i) * 1024 + lane * 16) = ca[u][i];
+#pragma unroll
+      for (int i = 0; i < B_CH; ++i) *(i32x4_t*)(sB(buf) + (wave * B_CH + i) * 1024 + lane * 16) = cb[u][i];
+    };
+#pragma unroll
+    for (int u = 0; u < PF; ++u)
+      if (u < nst) load_stage(u, u);
+    store_stage(0, 0);
+    if (PF < nst) load_stage(PF, 0);
+    __syncthreads();
+    for (int s0 = 0; s0 < nst; s0 += PF)
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        const int s = s0 + u;
+        if (s >= nst) break;  // uniform
+#pragma unroll
+        for (int kk = 0; kk < KST; ++kk) {
+          read_frags(s & 1, kk, kk & 1);
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = M::mma(fb[kk & 1][j], fa[kk & 1][i], acc[i][j]);
+        }
+        if (s + 1 < nst) {
+          store_stage((s + 1) & 1, (u + 1) % PF);  // that buffer was last read before the previous barrier
+          if (s + 1 + PF < nst) load_stage(s + 1 + PF, (u + 1) % PF);
+        }
+        // The stores above are LDS only: the loads in flight need no wait at the barrier.
+        __builtin_amdgcn_s_waitcnt(waitcnt_lgkm0);
+        __asm__ volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __asm__ volatile("" ::: "memory");
+      }
+  } else {
 #pragma unroll
   for (int st = 0; st < NS; ++st)
     if (st < nst) issue_rng(st, 0, PER, false);
@@ -463,6 +545,7 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   if (nst > 0) stage(s++, false);
   for (; s + NS + 2 <= nst; ++s) stage(s, true);
   for (; s < nst; ++s) stage(s, false);
+  }
 
   if (g.splits > 1 && !combine_splits<TM * TN, 64 * W>(g, batch * ntiles + tile, split, &acc[0][0])) return;
 
@@ -996,7 +1079,7 @@ void gemm4_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, 
   FO_HIP(hipGetLastError());
 }
 
-template <int KIND, int OUT, int BM, int BN, int WM, int WN, int NS>
+template <int KIND, int OUT, int BM, int BN, int WM, int WN, int NS, bool DMA = true>
 void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, const void* b, const float* scale,
                      int32_t* acc_out, int splits = 1, const GemmWorkspace* ws = nullptr) {
   GemmArgs g = gemm_args(d, c, a, b, scale, acc_out, BM, BN);
@@ -1009,12 +1092,12 @@ void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, c
   constexpr size_t lds = (size_t)NS * (BM + BN) * kRB;
   static bool attr_set = false;  // gfx950 LDS is 160 KiB; dynamic LDS above 64 KiB must be opted into
   if (!attr_set) {
-    FO_HIP(hipFuncSetAttribute((const void*)k_gemm<KIND, OUT, BM, BN, WM, WN, NS>,
+    FO_HIP(hipFuncSetAttribute((const void*)k_gemm<KIND, OUT, BM, BN, WM, WN, NS, DMA>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_set = true;
   }
   dim3 grid((unsigned)(tiles * splits), (unsigned)d.batch);
-  hipLaunchKernelGGL((k_gemm<KIND, OUT, BM, BN, WM, WN, NS>), grid, dim3(64 * WM * WN), lds, s, g);
+  hipLaunchKernelGGL((k_gemm<KIND, OUT, BM, BN, WM, WN, NS, DMA>), grid, dim3(64 * WM * WN), lds, s, g);
   FO_HIP(hipGetLastError());
 }
 
@@ -1039,6 +1122,31 @@ void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, c
 // against 32.7; with 8 stages left a split measured slower (16, 1024, 1024: 7.9 against 7.2).
 // FO_GEMM_TILE overrides the tile for measurement: 64, 128, 1284 (128x128, four stages), 2568 (k_gemm,
 // 256x256) or 4128 (k_gemm4).
+int64_t tiles_of(const GemmDesc& d, int64_t t) { return ((d.M + t - 1) / t) * ((d.N + t - 1) / t) * d.batch; }
+
+int splits_of(int64_t tiles, int64_t k_bytes) {
+  static_assert(GemmWorkspace::kTiles >= 256, "split workspace");
+  const int64_t stages = (k_bytes + kRB - 1) / kRB;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({256 / std::max<int64_t>(tiles, 1), stages / 12, 8}));
+}
+
+// Operands of any element alignment, with at least 8 rows and columns (fewer keep the exact vector-unit
+// fold, as aligned ones of several wheels do). The vector-unit fold took these before, per call: 333,
+// 1000, 777 bf16 -> f32 52.9 us against 8.9 here (relative error against 64 bits 2.1e-7 against 1.6e-7);
+// 71, 1928, 3677 234 us against 16.4 (5.7e-7 against 1.8e-7); 282, 5345, 521 bf16 86 against 15.4.
+template <int KIND, int OUT>
+void gemm_any_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, void* c, const void* a, const void* b) {
+  static int forced = [] {
+    const char* e = getenv("FO_GEMM_TILE");
+    return e ? atoi(e) : 0;
+  }();
+  const int64_t t64 = tiles_of(d, 64);
+  if (forced ? forced == 64 : t64 <= 512)
+    return gemm_launch_cfg<KIND, OUT, 64, 64, 2, 2, 2, false>(s, d, c, a, b, nullptr, nullptr,
+                                                              splits_of(t64, d.K * MfmaT<KIND>::EB), &ws);
+  gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 2, false>(s, d, c, a, b, nullptr, nullptr);
+}
+
 template <int KIND, int OUT>
 void gemm_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, void* c, const void* a, const void* b,
                  const float* scale = nullptr, int32_t* acc_out = nullptr) {
@@ -1047,23 +1155,18 @@ void gemm_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, void
     return e ? atoi(e) : 0;
   }();
   constexpr bool k16 = (KIND == kBf16 || KIND == kI8) && OUT <= 4;  // kinds with a 16x16 MFMA form here
-  auto tiles = [&](int64_t t) { return ((d.M + t - 1) / t) * ((d.N + t - 1) / t) * d.batch; };
-  const int64_t t64 = tiles(64);
+  const int64_t t64 = tiles_of(d, 64);
   int choice = forced;
-  if (!choice) choice = t64 <= 512 ? 64 : tiles(128) <= 256 ? 1284 : tiles(256) < 144 ? 128 : k16 ? 4128 : 2568;
+  if (!choice) choice = t64 <= 512 ? 64 : tiles_of(d, 128) <= 256 ? 1284 : tiles_of(d, 256) < 144 ? 128 : k16 ? 4128 : 2568;
   if constexpr (k16) {
     // four waves of 128x128 (16x16 MFMA tiles), 128-byte stages, A and B double-buffered. (A
     // triple-buffered, running a stage further ahead than B in the 32 KiB of LDS left over, measured
     // 1030-1034 against 1300-1307 TFLOP/s on one box: correct, and slower.)
     if (choice == 4128) return gemm4_launch_cfg<KIND, OUT, 2>(s, d, c, a, b, scale, acc_out);
   }
-  if (choice == 64) {
-    const int64_t stages = (d.K * MfmaT<KIND>::EB + kRB - 1) / kRB;
-    int64_t splits = std::min<int64_t>({256 / std::max<int64_t>(t64, 1), stages / 12, 8});
-    if (splits < 1) splits = 1;
-    static_assert(GemmWorkspace::kTiles >= 256, "split workspace");
-    return gemm_launch_cfg<KIND, OUT, 64, 64, 2, 2, 4>(s, d, c, a, b, scale, acc_out, (int)splits, &ws);
-  }
+  if (choice == 64)
+    return gemm_launch_cfg<KIND, OUT, 64, 64, 2, 2, 4>(s, d, c, a, b, scale, acc_out,
+                                                       splits_of(t64, d.K * MfmaT<KIND>::EB), &ws);
   if (choice == 1284) return gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 4>(s, d, c, a, b, scale, acc_out);
   if (choice == 128) return gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 2>(s, d, c, a, b, scale, acc_out);
   return gemm_launch_cfg<KIND, OUT, 256, 256, 2, 4, 2>(s, d, c, a, b, scale, acc_out);
@@ -1097,6 +1200,17 @@ void launch_gemm(hipStream_t s, void* c, const void* a, const void* b, fo_dtype 
   if (in_t == FO_F8E5M2 && out_t == FO_F8E5M2) return gemm_launch<kF8E5M2, 6>(s, d, ws, c, a, b);
   if (in_t == FO_F8E5M2 && out_t == FO_F32) return gemm_launch<kF8E5M2, 1>(s, d, ws, c, a, b);
   throw InvalidArg("gemm: unsupported dtype pair");
+}
+
+bool launch_gemm_any(hipStream_t s, void* c, const void* a, const void* b, fo_dtype in_t, fo_dtype out_t,
+                     const GemmDesc& d, const GemmWorkspace& ws) {
+  if (d.M < 8 || d.N < 8 || d.K <= 0 || d.M >= (1ll << 31) || d.N >= (1ll << 31) || d.batch <= 0 || d.batch >= 65536) return false;
+  if (d.K * 2 >= (1ll << 31) || 128 * std::max(d.lda, d.ldb) * 2 >= (1ll << 32)) return false;  // 32-bit offsets in a tile
+  if (in_t == FO_BF16 && out_t == FO_BF16) return gemm_any_launch<kBf16, 0>(s, d, ws, c, a, b), true;
+  if (in_t == FO_BF16 && out_t == FO_F32) return gemm_any_launch<kBf16, 1>(s, d, ws, c, a, b), true;
+  if (in_t == FO_I8 && out_t == FO_I8) return gemm_any_launch<kI8, 2>(s, d, ws, c, a, b), true;
+  if (in_t == FO_I8 && out_t == FO_I32) return gemm_any_launch<kI8, 3>(s, d, ws, c, a, b), true;
+  return false;
 }
 
 void launch_w8a8(hipStream_t s, uint16_t* out, int32_t* acc_out, const int8_t* a, const int8_t* w, const float* scale,

@@ -339,6 +339,9 @@ void launch_gemv(hipStream_t s, void* out, const void* x, const void* w, fo_dtyp
                  int64_t K, int64_t ldw, int64_t ldo, bool x_f32 = false);
 void launch_gemm(hipStream_t s, void* c, const void* a, const void* b, fo_dtype in_t, fo_dtype out_t,
                  const GemmDesc& d, const GemmWorkspace& ws);
+// The same contraction for operands of any element alignment (bf16 and i8); false when it does not take it.
+bool launch_gemm_any(hipStream_t s, void* c, const void* a, const void* b, fo_dtype in_t, fo_dtype out_t,
+                     const GemmDesc& d, const GemmWorkspace& ws);
 bool gemm_supported(fo_dtype in_t, fo_dtype out_t);
 bool gemm_aligned(const void* a, const void* b, fo_dtype in_t, const GemmDesc& d);
 
