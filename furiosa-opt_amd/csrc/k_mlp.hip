@@ -4,10 +4,13 @@
 // to bf16; bias add narrowed to bf16 (:164-176); argmax with the last maximum winning ties under
 // f32::total_cmp (tests/mnist_tests.rs:41-48).
 //
-// Latency-bound (13 MFLOP): one workgroup per batch row keeps the whole chain on chip. Each dot
-// product is one thread folding k in ascending order with separate multiply/add roundings -- the
-// emulator's own fold order -- so the logits match it bit for bit.
+// Latency-bound (13 MFLOP) at the example's batch of 64: one workgroup per batch row keeps the whole
+// chain on chip; larger batches share a workgroup's weights among rows. Each dot product is one thread
+// folding k in ascending order with separate multiply/add roundings -- the emulator's own fold order --
+// so the logits match it bit for bit.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "runtime.hpp"
 
@@ -269,6 +272,216 @@ __global__ void __launch_bounds__(kMlpThreads) k_mlp_split(int32_t* __restrict__
   }
 }
 
+// Any shape, and batches past one row a CU: a block of 512 threads carries R batch rows through both
+// layers. A thread owns one unit and RT of the block's rows: acc[r] = RN(acc[r] + RN(x[r][k] * w[k])), k
+// ascending, the emulator's own fold. Weights go through LDS as bf16 bits (subnormals already read as
+// zero), 32 k at a time, double-buffered, the 16-byte loads (any address) of the next two chunks in
+// flight; each weight is read once per block instead of once per row. Bound by the multiplies and adds
+// when RT is large (4096 x 784 x 128: 45 us against 21 us of them on every SIMD), by each chunk's chain of
+// LDS reads, serial adds, LDS writes and barrier (0.53 us) when it is 1.
+constexpr int kRowsT = 512;      // threads
+constexpr int kRowsKC = 32;      // k per chunk
+constexpr int kRowsPF = 2;       // chunks of weights in registers ahead of the two in LDS
+constexpr int kRowsPitch = 40;   // bf16 per LDS weight row: 16-byte reads of consecutive rows hit distinct banks
+typedef uint16_t u16x8_t __attribute__((ext_vector_type(8)));
+typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4_t;
+typedef i32x4_t i32x4_any_t __attribute__((aligned(2)));
+
+struct MlpArgs {
+  int32_t* pred;
+  uint16_t* logits;
+  const uint16_t *x, *w1, *b1, *w2, *b2;
+  int32_t batch, in_f, hidden, out_f;
+  int32_t xp, hp, op, wrows;  // LDS row pitches (floats), weight rows per buffer
+};
+
+// Weight rows a layer of n units stages at once, a power of two.
+__host__ __device__ __forceinline__ int layer_units(int n) {
+  int t = 16;
+  while (t < n && t < kRowsT) t *= 2;
+  return t;
+}
+
+// One layer for rows [rg * RT, rg * RT + RT) of the block: emit(row, unit, sum).
+template <int RT, typename F>
+__device__ __forceinline__ void fold_layer(const float* in, int pitch, const uint16_t* __restrict__ w, int K, int N, int HT,
+                                           int rows, uint16_t* wbuf, F&& emit) {
+  typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+  const int tid = threadIdx.x, hl = tid % HT, r0 = tid / HT * RT;
+  const int loads = HT * 4 / kRowsT > 0 ? HT * 4 / kRowsT : 1;  // chunk loads per thread, at most 4
+  const int nch = (K + kRowsKC - 1) / kRowsKC;
+  for (int n0 = 0; n0 < N; n0 += HT) {
+    // Thread's weight pieces: unit n0 + id / 4 (the last unit where it is past the layer: its sum is not
+    // used), k 8 (id % 4) .. + 7 of the chunk, for id = tid + j * threads.
+    i32x4_t wr[kRowsPF][4];
+    const uint16_t* wp[4];
+    bool has[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int id = tid + j * kRowsT;
+      has[j] = id < HT * 4;
+      wp[j] = w + (int64_t)min(n0 + id / 4, N - 1) * K + id % 4 * 8;
+    }
+    auto load = [&](int c, int u) __attribute__((always_inline)) {
+      const int k = c * kRowsKC;
+      if (k + kRowsKC <= K) {  // uniform
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j < loads && has[j]) wr[u][j] = *(const i32x4_any_t*)(wp[j] + k);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          u16x8_t v = (u16x8_t)(uint16_t)0;
+          const int at = k + (tid + j * kRowsT) % 4 * 8;
+          if (j < loads && has[j])
+            for (int e = 0; e < 8; ++e)
+              if (at + e < K) v[e] = wp[j][k + e];
+          wr[u][j] = __builtin_bit_cast(i32x4_t, v);
+        }
+      }
+    };
+    auto store = [&](int buf, int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j >= loads || !has[j]) continue;
+        const int id = tid + j * kRowsT;
+        i32x4_t v = wr[u][j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {  // both halves of a word: a zero exponent leaves the sign alone
+          const uint32_t q = (uint32_t)v[e], nz = ((q & 0x7f807f80u) + 0x7f807f80u) & 0x80008000u;
+          v[e] = (int)(q & ((nz - (nz >> 15)) | 0x80008000u));
+        }
+        *(i32x4_t*)(wbuf + (buf * HT + id / 4) * kRowsPitch + id % 4 * 8) = v;
+      }
+    };
+    float acc[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int u = 0; u < kRowsPF; ++u)
+      if (u < nch) load(u, u);
+    store(0, 0);
+    if (kRowsPF < nch) load(kRowsPF, 0);
+    __syncthreads();
+    for (int c0 = 0; c0 < nch; c0 += kRowsPF)
+#pragma unroll
+      for (int u = 0; u < kRowsPF; ++u) {
+        const int c = c0 + u;
+        if (c >= nch) break;  // uniform
+        if (r0 < rows) {
+          const uint16_t* wrow = wbuf + ((c & 1) * HT + hl) * kRowsPitch;
+          const float* xr = in + r0 * pitch + c * kRowsKC;
+          // A chunk's weights, and (RT rows at a time) its inputs, are read ahead of the adds: one LDS
+          // latency per batch of reads rather than one per eight adds.
+          constexpr int G = kRowsKC / 4, B = RT <= 2 ? G / RT : RT == 4 ? 2 : 1;  // 4-k groups per batch
+          u16x8_t q[G / 2];
+#pragma unroll
+          for (int g = 0; g < G / 2; ++g) q[g] = *(const u16x8_t*)(wrow + g * 8);
+#pragma unroll
+          for (int g0 = 0; g0 < G; g0 += B) {
+            f32x4_t xv[B][RT];
+#pragma unroll
+            for (int g = 0; g < B; ++g)
+#pragma unroll
+              for (int r = 0; r < RT; ++r) xv[g][r] = *(const f32x4_t*)(xr + r * pitch + (g0 + g) * 4);
+            if (RT <= 2) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < B; ++g)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int k = (g0 + g) * 4 + e;
+                const float wf = __uint_as_float((uint32_t)q[k / 8][k % 8] << 16);
+#pragma unroll
+                for (int r = 0; r < RT; ++r) acc[r] = __fadd_rn(acc[r], __fmul_rn(xv[g][r][e], wf));
+              }
+          }
+        }
+        if (c + 1 < nch) {
+          store((c + 1) & 1, (u + 1) % kRowsPF);  // that buffer was last read before the previous barrier
+          if (c + 1 + kRowsPF < nch) load(c + 1 + kRowsPF, (u + 1) % kRowsPF);
+        }
+        // An LDS-only barrier: the weight loads stay in flight across it.
+        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+        __asm__ volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __asm__ volatile("" ::: "memory");
+      }
+    if (r0 < rows && n0 + hl < N)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) emit(r0 + r, n0 + hl, acc[r]);
+  }
+}
+
+template <int R, typename F>
+__device__ __forceinline__ void fold_rows(const float* in, int pitch, const uint16_t* w, int K, int N, uint16_t* wbuf, F&& emit) {
+  const int HT = layer_units(N), rt = R * HT / kRowsT;  // rows per thread (R over 512 / HT row groups)
+  if (R >= 16 && rt == 16) return fold_layer<16>(in, pitch, w, K, N, HT, R, wbuf, emit);
+  if (R >= 8 && rt == 8) return fold_layer<8>(in, pitch, w, K, N, HT, R, wbuf, emit);
+  if (R >= 4 && rt == 4) return fold_layer<4>(in, pitch, w, K, N, HT, R, wbuf, emit);
+  if (R >= 2 && rt == 2) return fold_layer<2>(in, pitch, w, K, N, HT, R, wbuf, emit);
+  fold_layer<1>(in, pitch, w, K, N, HT, R, wbuf, emit);
+}
+
+template <int R>
+__global__ void __launch_bounds__(kRowsT) k_mlp_rows(MlpArgs g) {
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  float* xs = smem;
+  float* hs = xs + R * g.xp;
+  float* ys = hs + R * g.hp;
+  uint16_t* wbuf = (uint16_t*)(ys + R * g.op);
+  const int tid = threadIdx.x;
+  const int64_t b0 = (int64_t)blockIdx.x * R;
+  for (int i = tid; i < R * g.xp; i += kRowsT) {
+    const int r = i / g.xp, k = i - r * g.xp;
+    xs[i] = k < g.in_f && b0 + r < g.batch ? bf16_to_f32(g.x[(b0 + r) * g.in_f + k]) : 0.f;
+  }
+  for (int i = tid; i < R * g.hp; i += kRowsT) hs[i] = 0.f;  // also past `hidden`: the last chunk's tail
+  // (both are read after the first barrier in fold_layer)
+  fold_rows<R>(xs, g.xp, g.w1, g.in_f, g.hidden, wbuf, [&](int r, int h, float acc) __attribute__((always_inline)) {
+    const float hv = bf16_to_f32(f32_to_bf16(acc));                           // contract_lane + cast
+    const float z = fmaxf(__fadd_rn(hv, bf16_to_f32(g.b1[h])), 0.0f);         // clip Add, clip Max 0
+    hs[r * g.hp + h] = bf16_to_f32(f32_to_bf16(z));
+  });
+  __syncthreads();
+  fold_rows<R>(hs, g.hp, g.w2, g.hidden, g.out_f, wbuf, [&](int r, int o, float acc) __attribute__((always_inline)) {
+    const float yv = bf16_to_f32(f32_to_bf16(acc));
+    const uint16_t y = f32_to_bf16(__fadd_rn(yv, bf16_to_f32(g.b2[o])));
+    ys[r * g.op + o] = bf16_to_f32(y);
+    if (g.logits && b0 + r < g.batch) g.logits[(b0 + r) * g.out_f + o] = y;
+  });
+  __syncthreads();
+  if (tid < R && b0 + tid < g.batch) {
+    int best = 0;
+    int32_t bk = total_key(ys[tid * g.op]);
+    for (int o = 1; o < g.out_f; ++o) {
+      const int32_t kk = total_key(ys[tid * g.op + o]);
+      if (kk >= bk) {  // max_by keeps the last of equal maxima
+        bk = kk;
+        best = o;
+      }
+    }
+    g.pred[b0 + tid] = best;
+  }
+}
+
+template <int R>
+bool mlp_rows_launch(hipStream_t s, MlpArgs g) {
+  g.xp = (g.in_f + kRowsKC - 1) / kRowsKC * kRowsKC;
+  g.hp = (g.hidden + kRowsKC - 1) / kRowsKC * kRowsKC;
+  g.op = (g.out_f + 3) / 4 * 4;
+  g.wrows = std::max(layer_units(g.hidden), layer_units(g.out_f));
+  const size_t lds = (size_t)R * ((size_t)g.xp + g.hp + g.op) * 4 + (size_t)2 * g.wrows * kRowsPitch * 2;
+  if (lds > 160 * 1024) return false;
+  static bool attr_set = false;
+  if (!attr_set) {
+    FO_HIP(hipFuncSetAttribute((const void*)k_mlp_rows<R>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(k_mlp_rows<R>, dim3((unsigned)((g.batch + R - 1) / R)), dim3(kRowsT), lds, s, g);
+  FO_HIP(hipGetLastError());
+  return true;
+}
+
 }  // namespace
 
 void launch_mlp(hipStream_t s, int32_t* pred, uint16_t* logits, const uint16_t* x, const uint16_t* w1,
@@ -278,9 +491,29 @@ void launch_mlp(hipStream_t s, int32_t* pred, uint16_t* logits, const uint16_t* 
   const size_t lds_split =
       (size_t)(((in_f + 3) / 4 + (hidden + 3) / 4 + (out_f + 3) / 4) * 4 + 2 * hidden * kPP) * sizeof(float);
   const int64_t producers = kMlpThreads - (hidden + 63) / 64 * 64;
-  if (in_f % 8 == 0 && hidden <= 256 && hidden * (kKC / 8) <= kUnits * producers && out_f * ((hidden + 3) / 4 * 4) <= 2 * hidden * kPP &&
-      out_f * hidden <= kW2Per * kMlpThreads &&
-      ((uintptr_t)w1 % 16) == 0 && lds_split <= 160 * 1024) {
+  const bool split = in_f % 8 == 0 && hidden <= 256 && hidden * (kKC / 8) <= kUnits * producers &&
+                     out_f * ((hidden + 3) / 4 * 4) <= 2 * hidden * kPP && out_f * hidden <= kW2Per * kMlpThreads &&
+                     ((uintptr_t)w1 % 16) == 0 && lds_split <= 160 * 1024;
+  const size_t lds = (size_t)(in_f + hidden + out_f) * sizeof(float);
+  require(split || lds <= 64 * 1024, "mlp: layer widths exceed the LDS budget");
+  // A row per block while every row can have a CU: producers and folders (k_mlp_split) where the shape
+  // fits them. Past 256 rows, the fewest rows a block (a power of two) that leave one block a CU. Kernel
+  // alone in a recorded graph, batch x inputs x hidden x outputs, us, before -> k_mlp_rows:
+  //     256 x 784 x 128 x 10      14.6 (split) -> 23      4096 x 784 x 128 x 10     184 (split) -> 45
+  //     512 x 784 x 128 x 10      26.5 (split) -> 24      1104 x 270 x 147 x 33    32.6 (k_mlp) -> 24
+  //     1024 x 784 x 128 x 10     49.5 (split) -> 28      4096 x 1024 x 512 x 64    955 (k_mlp) -> 185
+  //     59 x 271 x 401 x 64       40.3 (k_mlp) -> 28      2 x 73 x 23 x 34          7.3 (k_mlp) -> 8.8
+  // so small layers the producers do not take keep a thread per fold (k_mlp).
+  const bool small = batch <= 256 && hidden <= 256 && in_f + hidden <= 128;
+  if (!(split && batch <= 256) && !small) {
+    MlpArgs g{pred, logits, x, w1, b1, w2, b2, (int32_t)batch, (int32_t)in_f, (int32_t)hidden, (int32_t)out_f, 0, 0, 0, 0};
+    if (batch > 2048 && mlp_rows_launch<16>(s, g)) return;
+    if (batch > 1024 && mlp_rows_launch<8>(s, g)) return;
+    if (batch > 512 && mlp_rows_launch<4>(s, g)) return;
+    if (batch > 256 && mlp_rows_launch<2>(s, g)) return;
+    if (mlp_rows_launch<1>(s, g)) return;
+  }
+  if (split) {
     static bool attr_set = false;  // dynamic LDS above 64 KiB must be opted into
     if (!attr_set) {
       FO_HIP(hipFuncSetAttribute((const void*)k_mlp_split, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
@@ -288,13 +521,10 @@ void launch_mlp(hipStream_t s, int32_t* pred, uint16_t* logits, const uint16_t* 
     }
     hipLaunchKernelGGL(k_mlp_split, dim3((unsigned)batch), dim3(kMlpThreads), lds_split, s, pred, logits, x, w1, b1, w2,
                        b2, (int32_t)in_f, (int32_t)hidden, (int32_t)out_f);
-    FO_HIP(hipGetLastError());
-    return;
+  } else {
+    hipLaunchKernelGGL(k_mlp, dim3((unsigned)batch), dim3(256), lds, s, pred, logits, x, w1, b1, w2, b2, (int32_t)in_f,
+                       (int32_t)hidden, (int32_t)out_f);
   }
-  size_t lds = (size_t)(in_f + hidden + out_f) * sizeof(float);
-  require(lds <= 64 * 1024, "mlp: layer widths exceed the LDS budget");
-  hipLaunchKernelGGL(k_mlp, dim3((unsigned)batch), dim3(256), lds, s, pred, logits, x, w1, b1, w2, b2, (int32_t)in_f,
-                     (int32_t)hidden, (int32_t)out_f);
   FO_HIP(hipGetLastError());
 }
 
