@@ -11,6 +11,8 @@
 // both sides and the dtype / op switches are wave-uniform branches around register work.
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 #include "runtime.hpp"
 
 namespace fo {
@@ -532,6 +534,193 @@ __global__ void __launch_bounds__(kBlock) k_map_w(void* __restrict__ dst, const 
   }
 }
 
+// ---- small elementwise passes ---------------------------------------------------------------------
+//
+// The decode step's maps and zips are chains of dependent launches over a few thousand elements or
+// fewer, bound by latency: the launch, the instruction fetches of a cold kernel and one memory round
+// trip. These forms take one element a lane and are built per op, so a kernel is a few straight cache lines
+// of code (the general forms carry every op's code, dispatched per element for zips, and lanes that
+// work through 8 elements in turn).
+constexpr uint64_t kSmall = 32768;  // elements (zips and maps alike)
+constexpr int kSmallBlock = 64;
+
+enum SmallOp { kAdd, kSub, kMul, kDiv, kMin, kMax, kExp, kNegExp, kSqrt, kSigmoid, kNone };
+
+// The float ops with a small form; kNone for the rest. A swapped op is the caller's to turn around.
+SmallOp small_binary(int code) {
+  switch (code) {
+    case FO_OP_ADD_F:
+    case FO_OP_CLIP_ADD: return kAdd;
+    case FO_OP_SUB_F: return kSub;
+    case FO_OP_MUL_F: return kMul;
+    case FO_OP_DIV_F: return kDiv;
+    case FO_OP_CLIP_MIN: return kMin;
+    case FO_OP_CLIP_MAX: return kMax;
+  }
+  return kNone;
+}
+SmallOp small_unary(int code) {
+  switch (code) {
+    case FO_OP_EXP: return kExp;
+    case FO_OP_NEG_EXP: return kNegExp;
+    case FO_OP_SQRT: return kSqrt;
+    case FO_OP_SIGMOID: return kSigmoid;
+  }
+  return kNone;
+}
+// The same expressions as binary_op and unary_op.
+template <int OP>
+__device__ __forceinline__ float small_op(float a, float b) {
+  if constexpr (OP == kAdd) return __fadd_rn(a, b);
+  if constexpr (OP == kSub) return __fsub_rn(a, b);
+  if constexpr (OP == kMul) return __fmul_rn(a, b);
+  if constexpr (OP == kDiv) return __fdiv_rn(a, b);
+  if constexpr (OP == kMin) return fminf(a, b);
+  if constexpr (OP == kMax) return fmaxf(a, b);
+  if constexpr (OP == kExp) return expf(a);
+  if constexpr (OP == kNegExp) return expf(-a);
+  if constexpr (OP == kSqrt) return sqrt_rn(a);
+  return __fdiv_rn(1.0f, __fadd_rn(1.0f, expf(-a)));  // kSigmoid
+}
+
+// A deferred map applied on load: an immediate op (reversed: imm op x) or a unary one.
+struct SmallPre {
+  int32_t n = 0;
+  int32_t op[3] = {};
+  int32_t swap[3] = {};
+  float imm[3] = {};
+};
+bool small_pre(const PreOps& in, SmallPre* out) {
+  out->n = in.n;
+  for (int k = 0; k < in.n; ++k) {
+    const SmallOp b = small_binary(in.op[k].code), u = small_unary(in.op[k].code);
+    if (b == kNone && u == kNone) return false;
+    out->op[k] = b != kNone ? b : u;
+    out->swap[k] = b != kNone && (in.op[k].flags & FO_OP_SWAP);
+    out->imm[k] = bits_f32(in.op[k].imm0);
+  }
+  return true;
+}
+struct SmallIn {
+  const void* p;
+  int32_t code;       // 4, 2 or kViaBf16, as in read_word
+  FastDiv div, mod;   // element i reads (i / div) % mod (mod.d 0: no wrap)
+  SmallPre pre;
+};
+
+template <bool PRE, bool BC>
+__device__ __forceinline__ float small_in(const SmallIn& in, uint32_t i) {
+  if constexpr (BC) {
+    i = in.div.div(i);
+    if (in.mod.d != 0) i -= in.mod.div(i) * in.mod.d;
+  }
+  float x = in.code == 2 ? bf16_to_f32(((const uint16_t*)in.p)[i]) : ((const float*)in.p)[i];
+  if constexpr (PRE) {
+    for (int k = 0; k < in.pre.n; ++k) {
+      const float a = in.pre.swap[k] ? in.pre.imm[k] : x, b = in.pre.swap[k] ? x : in.pre.imm[k];
+      switch (in.pre.op[k]) {
+        case kAdd: x = small_op<kAdd>(a, b); break;
+        case kSub: x = small_op<kSub>(a, b); break;
+        case kMul: x = small_op<kMul>(a, b); break;
+        case kDiv: x = small_op<kDiv>(a, b); break;
+        case kMin: x = small_op<kMin>(a, b); break;
+        case kMax: x = small_op<kMax>(a, b); break;
+        case kExp: x = small_op<kExp>(x, x); break;
+        case kNegExp: x = small_op<kNegExp>(x, x); break;
+        case kSqrt: x = small_op<kSqrt>(x, x); break;
+        default: x = small_op<kSigmoid>(x, x); break;
+      }
+    }
+  }
+  return in.code == kViaBf16 ? bf16_to_f32(f32_to_bf16(x)) : x;
+}
+
+template <int OP, bool PRE, bool BC>
+__global__ void __launch_bounds__(kSmallBlock) k_zip_small(float* __restrict__ dst, SmallIn a, SmallIn b, uint32_t n) {
+  const uint32_t i = blockIdx.x * kSmallBlock + threadIdx.x;
+  if (i >= n) return;
+  const float x = small_in<PRE, BC>(a, i), y = small_in<PRE, BC>(b, i);
+  dst[i] = small_op<OP>(x, y);
+}
+
+template <bool PRE, bool BC>
+bool zip_small_op(hipStream_t s, SmallOp op, void* dst, const SmallIn& a, const SmallIn& b, uint32_t n) {
+  const dim3 grid((n + kSmallBlock - 1) / kSmallBlock), block(kSmallBlock);
+  switch (op) {
+    case kAdd: hipLaunchKernelGGL((k_zip_small<kAdd, PRE, BC>), grid, block, 0, s, (float*)dst, a, b, n); break;
+    case kSub: hipLaunchKernelGGL((k_zip_small<kSub, PRE, BC>), grid, block, 0, s, (float*)dst, a, b, n); break;
+    case kMul: hipLaunchKernelGGL((k_zip_small<kMul, PRE, BC>), grid, block, 0, s, (float*)dst, a, b, n); break;
+    case kDiv: hipLaunchKernelGGL((k_zip_small<kDiv, PRE, BC>), grid, block, 0, s, (float*)dst, a, b, n); break;
+    case kMin: hipLaunchKernelGGL((k_zip_small<kMin, PRE, BC>), grid, block, 0, s, (float*)dst, a, b, n); break;
+    case kMax: hipLaunchKernelGGL((k_zip_small<kMax, PRE, BC>), grid, block, 0, s, (float*)dst, a, b, n); break;
+    default: return false;
+  }
+  FO_HIP(hipGetLastError());
+  return true;
+}
+
+// zip_with over f32 words (inputs as in launch_zip_bcast) by the small form; false when it has none.
+bool zip_small(hipStream_t s, void* dst, const void* a, int a_code, uint32_t a_div, uint32_t a_mod, const PreOps& a_pre,
+               const void* b, int b_code, uint32_t b_div, uint32_t b_mod, const PreOps& b_pre, uint64_t n, const fo_op& op) {
+  const SmallOp so = small_binary(op.code);
+  if (so == kNone || n == 0 || n > kSmall) return false;
+  SmallIn x{a, a_code, FastDiv(a_div), FastDiv(a_mod ? a_mod : 1), {}}, y{b, b_code, FastDiv(b_div), FastDiv(b_mod ? b_mod : 1), {}};
+  if (!a_mod) x.mod.d = 0;
+  if (!b_mod) y.mod.d = 0;
+  if (!small_pre(a_pre, &x.pre) || !small_pre(b_pre, &y.pre)) return false;
+  if (op.flags & FO_OP_SWAP) std::swap(x, y);
+  const bool pre = a_pre.n || b_pre.n, bc = a_div != 1 || a_mod || b_div != 1 || b_mod;
+  if (pre) return bc ? zip_small_op<true, true>(s, so, dst, x, y, (uint32_t)n) : zip_small_op<true, false>(s, so, dst, x, y, (uint32_t)n);
+  return bc ? zip_small_op<false, true>(s, so, dst, x, y, (uint32_t)n) : zip_small_op<false, false>(s, so, dst, x, y, (uint32_t)n);
+}
+
+// map of f32 words read by `code`: OP with the immediate (or unary), f32 out; OP kNone: the narrow to bf16.
+template <int OP>
+__global__ void __launch_bounds__(kSmallBlock) k_map_small(void* __restrict__ dst, const void* __restrict__ src, int32_t code,
+                                                     int32_t narrow, int32_t swap, float imm, uint32_t n) {
+  const uint32_t i = blockIdx.x * kSmallBlock + threadIdx.x;
+  if (i >= n) return;
+  float x = code == 2 ? bf16_to_f32(((const uint16_t*)src)[i]) : ((const float*)src)[i];
+  if (code == kViaBf16) x = bf16_to_f32(f32_to_bf16(x));
+  if constexpr (OP != kNone) x = small_op<OP>(swap ? imm : x, swap ? x : imm);
+  if (narrow)
+    ((uint16_t*)dst)[i] = f32_to_bf16(x);
+  else
+    ((float*)dst)[i] = x;
+}
+
+// map by the small form: f32 words (read code 4, 2 or kViaBf16) through a float op to f32, or the cast of
+// f32 to bf16; false when it has none.
+bool map_small(hipStream_t s, void* dst, fo_dtype dst_t, const void* src, int code, uint64_t n, const fo_op& op) {
+  if (n == 0 || n > kSmall) return false;
+  const dim3 grid((unsigned)((n + kSmallBlock - 1) / kSmallBlock)), block(kSmallBlock);
+  const SmallOp b = small_binary(op.code), u = small_unary(op.code);
+  const int swap = b != kNone && (op.flags & FO_OP_SWAP) ? 1 : 0;
+  const float imm = bits_f32(op.imm0);
+  const bool cast = op.code == FO_OP_CAST && dst_t == FO_BF16;
+  if (!cast && (dst_t != FO_F32 || (b == kNone && u == kNone))) return false;
+#define FO_SMALL(OP)                                                                                            \
+  case OP:                                                                                                      \
+    hipLaunchKernelGGL(k_map_small<OP>, grid, block, 0, s, dst, src, code, (int)cast, swap, imm, (uint32_t)n);   \
+    break
+  switch (cast ? kNone : b != kNone ? b : u) {
+    FO_SMALL(kAdd);
+    FO_SMALL(kSub);
+    FO_SMALL(kMul);
+    FO_SMALL(kDiv);
+    FO_SMALL(kMin);
+    FO_SMALL(kMax);
+    FO_SMALL(kExp);
+    FO_SMALL(kNegExp);
+    FO_SMALL(kSqrt);
+    FO_SMALL(kSigmoid);
+    FO_SMALL(kNone);
+  }
+#undef FO_SMALL
+  FO_HIP(hipGetLastError());
+  return true;
+}
+
 // ---- zip3 with tag-guarded slots (apply_slots) --------------------------------------------------
 // Each cell takes the first register slot whose guard admits its execution id, else the port slot
 // if its guard admits, else passes through. A tag byte above 15 is not an execution id (the
@@ -842,6 +1031,7 @@ void launch_map(hipStream_t s, void* dst, fo_dtype dst_t, const void* src, fo_dt
     require(!is_f8(src_t) && !is_f8(dst_t), "map: 8-bit floats take casts and table lookups only");
   }
   require(aligned16(dst) && aligned16(src), "map: buffers must be 16-byte aligned");
+  if (src_t == FO_F32 && map_small(s, dst, dst_t, src, 4, n, op)) return;
   const int sb = width_of(src_t), db = width_of(dst_t);
 #define FO_MAP_CASE(S, D)                                  \
   if (sb == S && db == D) {                                \
@@ -867,6 +1057,7 @@ void launch_zip(hipStream_t s, void* dst, fo_dtype dst_t, const void* a, const v
   require(in_t != FO_F8E4M3 && in_t != FO_F8E5M2 && dst_t != FO_F8E4M3 && dst_t != FO_F8E5M2,
           "zip_with: 8-bit floats take casts and table lookups only");
   require(aligned16(dst) && aligned16(a) && aligned16(b), "zip_with: buffers must be 16-byte aligned");
+  if (in_t == FO_F32 && dst_t == FO_F32 && zip_small(s, dst, a, 4, 1, 0, PreOps{}, b, 4, 1, 0, PreOps{}, n, op)) return;
   const int ib = width_of(in_t), ob = width_of(dst_t);
 #define FO_ZIP_CASE(I, O)                            \
   if (ib == I && ob == O) {                          \
@@ -892,6 +1083,7 @@ void launch_zip_widened(hipStream_t s, void* dst, fo_dtype dst_t, const void* a,
   require(dst_t == FO_F32, "zip_with: widened inputs take f32 outputs");
   require(a_pre.n >= 0 && a_pre.n <= 3 && b_pre.n >= 0 && b_pre.n <= 3, "zip_with: at most three deferred maps");
   require(aligned16(dst) && aligned16(a) && aligned16(b), "zip_with: buffers must be 16-byte aligned");
+  if (zip_small(s, dst, a, a_code, 1, 0, a_pre, b, b_code, 1, 0, b_pre, n, op)) return;
 #define FO_ZIPW_CASE(A, B)                                                                                     \
   if (a_code == A && b_code == B) {                                                                            \
     constexpr int MINB = code_bytes(A) < code_bytes(B) ? code_bytes(A) : code_bytes(B);                        \
@@ -923,6 +1115,7 @@ void launch_zip_bcast(hipStream_t s, void* dst, const void* a, int a_code, uint3
   require(a_div >= 1 && b_div >= 1, "zip_with: broadcast divisor must be positive");
   require(n < (1ull << 31), "zip_with: a broadcast input takes fewer than 2^31 elements");
   require(a_pre.n >= 0 && a_pre.n <= 3 && b_pre.n >= 0 && b_pre.n <= 3, "zip_with: at most three deferred maps");
+  if (zip_small(s, dst, a, a_code, a_div, a_mod, a_pre, b, b_code, b_div, b_mod, b_pre, n, op)) return;
   if (a_pre.n != 0 || b_pre.n != 0)
     hipLaunchKernelGGL(k_zip_b<true>, dim3(grid_for((int64_t)n)), dim3(kBlock), 0, s, (uint32_t*)dst,
                        ZipIn{a, a_code, a_div, a_mod, a_pre}, ZipIn{b, b_code, b_div, b_mod, b_pre}, n, op);
@@ -937,6 +1130,7 @@ void launch_map_widened(hipStream_t s, void* dst, fo_dtype dst_t, const void* sr
   require(aligned16(dst) && aligned16(src), "map: buffers must be 16-byte aligned");
   require(dst_t == FO_F32 || dst_t == FO_BF16, "map: a widened input takes f32 or bf16 outputs");
   require(src_code == 2 || src_code == kViaBf16, "map: unknown widened input code");
+  if (map_small(s, dst, dst_t, src, src_code, n, op)) return;
 #define FO_MAPW_CASE(SC, DB)                                                                                   \
   if (src_code == SC && (int)dtype_bytes(dst_t) == DB) {                                                       \
     constexpr int V = 16 / (code_bytes(SC) > DB ? code_bytes(SC) : DB);                                        \
