@@ -956,14 +956,17 @@ __global__ void __launch_bounds__(kBlock) k_reduce_thread(void* dst, const void*
 }
 
 // Thread per cell over a residue of one wheel (`total` elements `rstride` apart): the reads of a
-// batch are issued together and folded in order, the emulator's serial fold.
-template <typename Tag>
-__global__ void __launch_bounds__(kBlock) k_reduce_strided(void* dst, const void* src, int64_t src_len,
-                                                           uint32_t out_count, Wheels<1> ow, uint32_t total,
-                                                           int64_t rstride, int op, uint32_t identity) {
+// batch are issued together and folded in order, the emulator's serial fold. OP as in k_reduce_wave;
+// SAFE: every read is inside the source (no per-read checks). The small form (OP given, SAFE, one wave a
+// block, 32 reads in flight) serves the sum of 32 partial products.
+template <typename Tag, int OP, bool SAFE, int BLOCK>
+__global__ void __launch_bounds__(BLOCK) k_reduce_strided(void* dst, const void* src, int64_t src_len,
+                                                          uint32_t out_count, Wheels<1> ow, uint32_t total,
+                                                          int64_t rstride, int op_arg, uint32_t identity) {
   using R = RedT<Tag>;
-  constexpr int U = 16;
-  for (uint32_t o = blockIdx.x * kBlock + threadIdx.x; o < out_count; o += gridDim.x * kBlock) {
+  const int op = OP >= 0 ? OP : op_arg;
+  constexpr int U = SAFE ? 32 : 16;
+  for (uint32_t o = blockIdx.x * BLOCK + threadIdx.x; o < out_count; o += gridDim.x * BLOCK) {
     int64_t b[1];
     const bool dead = cell_base(ow, o, out_count, b);
     auto acc = R::from_bits(identity);
@@ -973,9 +976,10 @@ __global__ void __launch_bounds__(kBlock) k_reduce_strided(void* dst, const void
         bool ok[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int64_t off = b[0] + (int64_t)(r0 + u) * rstride;
-          ok[u] = r0 + u < total && off >= 0 && off < src_len;
-          v[u] = R::load(src, ok[u] ? off : 0);
+          ok[u] = r0 + u < total;
+          const int64_t off = b[0] + (int64_t)(SAFE && !ok[u] ? 0 : r0 + u) * rstride;
+          if (!SAFE) ok[u] = ok[u] && off >= 0 && off < src_len;
+          v[u] = R::load(src, SAFE || ok[u] ? off : 0);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -986,11 +990,15 @@ __global__ void __launch_bounds__(kBlock) k_reduce_strided(void* dst, const void
   }
 }
 
-template <typename Tag>
+// OP: the op as a constant (f32 sums and maxima, which the decode chains issue), or -1 for `op_arg`; CONTIG:
+// the residue is one contiguous run. A kernel built for its op and residue is a third of the code, and the
+// decode step's small reduces wait for instruction fetches as much as for data.
+template <typename Tag, int OP, bool CONTIG>
 __global__ void __launch_bounds__(kBlock) k_reduce_wave(void* dst, const void* src, int64_t src_len, uint32_t out_count,
-                                                        Wheels<1> ow, Wheels<1> rw, int op, uint32_t identity,
+                                                        Wheels<1> ow, Wheels<1> rw, int op_arg, uint32_t identity,
                                                         uint32_t neutral) {
   using R = RedT<Tag>;
+  const int op = OP >= 0 ? OP : op_arg;
   const int lane = threadIdx.x & 63;
   uint32_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
   uint32_t nwaves = (gridDim.x * kBlock) >> 6;
@@ -1010,7 +1018,7 @@ __global__ void __launch_bounds__(kBlock) k_reduce_wave(void* dst, const void* s
     // Each lane folds its strided slice from the op's neutral element, so the caller's identity
     // enters the result exactly once, after the lanes combine.
     auto acc = R::from_bits(neutral);
-    if (rw.n == 1 && rw.stride[0][0] == 1) {
+    if (CONTIG || (rw.n == 1 && rw.stride[0][0] == 1)) {
       // One contiguous residue run: 8 coalesced reads per lane in flight, no odometer.
       const int64_t lim = dead ? 0 : min((int64_t)total, src_len - base);
       int64_t r = lane;
@@ -1314,8 +1322,19 @@ void reduce_t(hipStream_t s, void* dst, const void* src, int64_t src_len, int64_
       break;
   }
   if (!exact_only && total >= 64 && res_contig && out_count <= (1 << 20)) {
-    hipLaunchKernelGGL(k_reduce_wave<Tag>, dim3(grid_for(out_count * 64)), dim3(kBlock), 0, s, dst, src, src_len,
-                       (uint32_t)out_count, ow, rw, op, identity, neutral);
+    const dim3 grid(grid_for(out_count * 64)), block(kBlock);
+    const bool run = is_f32 && rw.n == 1;  // one contiguous residue run
+    if constexpr (is_f32) {
+      if (run && op == FO_RED_ADD)
+        hipLaunchKernelGGL((k_reduce_wave<Tag, FO_RED_ADD, true>), grid, block, 0, s, dst, src, src_len,
+                           (uint32_t)out_count, ow, rw, op, identity, neutral);
+      else if (run && op == FO_RED_MAX)
+        hipLaunchKernelGGL((k_reduce_wave<Tag, FO_RED_MAX, true>), grid, block, 0, s, dst, src, src_len,
+                           (uint32_t)out_count, ow, rw, op, identity, neutral);
+    }
+    if (!(run && (op == FO_RED_ADD || op == FO_RED_MAX)))
+      hipLaunchKernelGGL((k_reduce_wave<Tag, -1, false>), grid, block, 0, s, dst, src, src_len, (uint32_t)out_count, ow, rw,
+                         op, identity, neutral);
   } else if (!exact_only && total >= 64 && cells_contig) {
     hipLaunchKernelGGL(k_reduce_cols<Tag>, dim3((unsigned)((out_count + 63) / 64)), dim3(64 * kSeg), 0, s, dst, src,
                        src_len, (uint32_t)out_count, ow, rw, op, identity, neutral, (uint32_t)total);
@@ -1325,8 +1344,22 @@ void reduce_t(hipStream_t s, void* dst, const void* src, int64_t src_len, int64_
     hipLaunchKernelGGL(k_reduce_tiled<Tag>, dim3((unsigned)blocks), dim3(256), 0, s, dst, src, src_len,
                        (uint32_t)out_count, ow, rw, op, identity, (uint32_t)total);
   } else if (rw.n == 1) {
-    hipLaunchKernelGGL(k_reduce_strided<Tag>, dim3(grid_for(out_count)), dim3(kBlock), 0, s, dst, src, src_len,
-                       (uint32_t)out_count, ow, (uint32_t)total, rw.stride[0][0], op, identity);
+    int64_t last = (total - 1) * rw.stride[0][0];
+    bool safe = rw.stride[0][0] >= 0 && total > 0;
+    for (int i = 0; i < ow.n; ++i) {
+      last += (int64_t)(ow.live[i] - 1) * ow.stride[0][i];
+      safe &= ow.stride[0][i] >= 0 && ow.live[i] > 0;
+    }
+    bool small = false;
+    if constexpr (is_f32) {
+      small = safe && last < src_len && op == FO_RED_ADD && out_count <= 32768;
+      if (small)
+        hipLaunchKernelGGL((k_reduce_strided<Tag, FO_RED_ADD, true, 64>), dim3((unsigned)((out_count + 63) / 64)), dim3(64), 0,
+                           s, dst, src, src_len, (uint32_t)out_count, ow, (uint32_t)total, rw.stride[0][0], op, identity);
+    }
+    if (!small)
+      hipLaunchKernelGGL((k_reduce_strided<Tag, -1, false, kBlock>), dim3(grid_for(out_count)), dim3(kBlock), 0, s, dst, src,
+                         src_len, (uint32_t)out_count, ow, (uint32_t)total, rw.stride[0][0], op, identity);
   } else {
     hipLaunchKernelGGL(k_reduce_thread<Tag>, dim3(grid_for(out_count)), dim3(kBlock), 0, s, dst, src, src_len,
                        (uint32_t)out_count, ow, rw, op, identity);
@@ -1910,6 +1943,50 @@ __global__ void __launch_bounds__(64 * kTileW) k_contract_tiled(Out* __restrict_
   }
 }
 
+// k_contract_generic for a residue of one wheel whose reads all lie inside the operands: no odometer and no
+// checks (11 KB of code become 3; the 65,536 sixteen-key partial products of an attention chunk). The same
+// fold in k order.
+template <typename In, typename Acc, typename Out>
+__global__ void __launch_bounds__(kBlock) k_contract_wheel(Out* __restrict__ out, const In* __restrict__ lhs,
+                                                           const In* __restrict__ rhs, uint32_t out_count, Wheels<2> ow,
+                                                           uint32_t total, int64_t sl, int64_t sr) {
+  using M = MacT<In, Acc>;
+  constexpr int U = 16;
+  const uint32_t o = blockIdx.x * kBlock + threadIdx.x;
+  if (o >= out_count) return;
+  int64_t b[2];
+  const bool dead = cell_base(ow, o, out_count, b);
+  Acc acc = Acc(0);
+  if (!dead) {  // a padding cell has no reads and keeps its zero
+    const In *pl = lhs + b[0], *pr = rhs + b[1];
+    for (uint32_t r0 = 0; r0 < total; r0 += U) {
+      In va[U], vb[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t r = r0 + u < total ? r0 + u : 0;
+        va[u] = pl[r * sl];
+        vb[u] = pr[r * sr];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (r0 + u < total) acc = M::mac(acc, M::widen(va[u]), M::widen(vb[u]));
+    }
+  }
+  out[o] = narrow<In, Acc, Out>(acc);
+}
+
+// Every read of the plan lies inside the operands.
+bool reads_inside(const Wheels<2>& ow, const Wheels<2>& rw, int64_t ll, int64_t rl) {
+  int64_t last[2] = {0, 0};
+  for (const Wheels<2>* w : {&ow, &rw})
+    for (int i = 0; i < w->n; ++i)
+      for (int k = 0; k < 2; ++k) {
+        if (w->live[i] == 0 || w->stride[k][i] < 0) return false;
+        last[k] += (int64_t)(w->live[i] - 1) * w->stride[k][i];
+      }
+  return last[0] < ll && last[1] < rl;
+}
+
 template <typename In, typename Acc, typename Out>
 void contract_t(hipStream_t s, void* out, const void* lhs, const void* rhs, int64_t ll, int64_t rl, int64_t n,
                 const Wheels<2>& ow, const Wheels<2>& rw) {
@@ -1923,6 +2000,10 @@ void contract_t(hipStream_t s, void* out, const void* lhs, const void* rhs, int6
     if (blocks > 65535ll * 16) blocks = 65535ll * 16;
     hipLaunchKernelGGL((k_contract_tiled<In, Acc, Out>), dim3((unsigned)blocks), dim3(64 * kTileW), 0, s, (Out*)out,
                        (const In*)lhs, (const In*)rhs, ll, rl, (uint32_t)n, ow, rw, (uint32_t)total);
+  } else if (rw.n == 1 && rw.live[0] == rw.size[0] && n < (1ll << 31) - kBlock && reads_inside(ow, rw, ll, rl)) {
+    hipLaunchKernelGGL((k_contract_wheel<In, Acc, Out>), dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
+                       (Out*)out, (const In*)lhs, (const In*)rhs, (uint32_t)n, ow, (uint32_t)total, rw.stride[0][0],
+                       rw.stride[1][0]);
   } else {
     hipLaunchKernelGGL((k_contract_generic<In, Acc, Out>), dim3(grid_for(n)), dim3(kBlock), 0, s, (Out*)out,
                        (const In*)lhs, (const In*)rhs, ll, rl, (uint32_t)n, ow, rw);
