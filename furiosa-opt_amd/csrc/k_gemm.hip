@@ -1116,18 +1116,29 @@ void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, c
 // for bf16 and i8, eight waves of 128x64 in 32x32 tiles (k_gemm) for the 8-bit floats, whose 32-byte
 // fragments have no 16x16 form here.
 //
-// Few 64x64 tiles leave CUs idle while each walks all of K, so up to 8 blocks share a tile while
-// that adds no second block to a CU and leaves each at least 12 stages (combine_splits costs about
-// 2.5 us): 64, 1024, 4096 in 10.6 us with 4 against 18.3 with one; 256, 256, 8192 in 13.2 with 8
-// against 32.7; with 8 stages left a split measured slower (16, 1024, 1024: 7.9 against 7.2).
-// FO_GEMM_TILE overrides the tile for measurement: 64, 128, 1284 (128x128, four stages), 2568 (k_gemm,
+// Up to 32 rows: 32x64 tiles of two waves, half the LDS traffic a stage (i8 16, 8192, 8192 15.8 us against
+// 18.0 for 64x64, bf16 16, 4096, 4096 11.9 against 13.6, each with its best number of blocks a tile).
+//
+// Few tiles leave CUs idle while each walks all of K, so blocks share a tile (splits_of): 64, 1024, 4096
+// in 10.6 us with 4 against 18.3 with one; 256, 256, 8192 in 13.2 with 8 against 32.7; but 256, 2048, 2048
+// 14.0 with 2 against 11.6 with one.
+// FO_GEMM_TILE overrides the tile for measurement: 32 (32x64), 64, 128, 1284 (128x128, four stages), 2568 (k_gemm,
 // 256x256) or 4128 (k_gemm4).
 int64_t tiles_of(const GemmDesc& d, int64_t t) { return ((d.M + t - 1) / t) * ((d.N + t - 1) / t) * d.batch; }
 
-int splits_of(int64_t tiles, int64_t k_bytes) {
+// Blocks sharing a tile of `rows` x 64, for the least estimated time: a stage of k takes 0.23 us when a
+// block has its CU to itself, sharing costs 2.2 us and, for the partial accumulators, 17 ns (64 rows) or
+// 9.5 ns (32) per block. At most one block a CU in all (the workspace is sized for it) and 8 a tile.
+int splits_of(int64_t tiles, int64_t k_bytes, int rows) {
   static_assert(GemmWorkspace::kTiles >= 256, "split workspace");
   const int64_t stages = (k_bytes + kRB - 1) / kRB;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({256 / std::max<int64_t>(tiles, 1), stages / 12, 8}));
+  int best = 1;
+  double least = 0.23 * (double)stages;
+  for (int s = 2; s <= 8 && s <= stages && s * tiles <= 256; ++s) {
+    const double t = 0.23 * (double)((stages + s - 1) / s) + 2.2 + (rows == 32 ? 0.0095 : 0.017) * (double)(s * tiles);
+    if (t < least) least = t, best = s;
+  }
+  return best;
 }
 
 // Operands of any element alignment, with at least 8 rows and columns (fewer keep the exact vector-unit
@@ -1143,7 +1154,7 @@ void gemm_any_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, 
   const int64_t t64 = tiles_of(d, 64);
   if (forced ? forced == 64 : t64 <= 512)
     return gemm_launch_cfg<KIND, OUT, 64, 64, 2, 2, 2, false>(s, d, c, a, b, nullptr, nullptr,
-                                                              splits_of(t64, d.K * MfmaT<KIND>::EB), &ws);
+                                                              splits_of(t64, d.K * MfmaT<KIND>::EB, 64), &ws);
   gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 2, false>(s, d, c, a, b, nullptr, nullptr);
 }
 
@@ -1157,16 +1168,19 @@ void gemm_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, void
   constexpr bool k16 = (KIND == kBf16 || KIND == kI8) && OUT <= 4;  // kinds with a 16x16 MFMA form here
   const int64_t t64 = tiles_of(d, 64);
   int choice = forced;
-  if (!choice) choice = t64 <= 512 ? 64 : tiles_of(d, 128) <= 256 ? 1284 : tiles_of(d, 256) < 144 ? 128 : k16 ? 4128 : 2568;
+  if (!choice) choice = d.M <= 32 && t64 <= 512 ? 32 : t64 <= 512 ? 64 : tiles_of(d, 128) <= 256 ? 1284 : tiles_of(d, 256) < 144 ? 128 : k16 ? 4128 : 2568;
   if constexpr (k16) {
     // four waves of 128x128 (16x16 MFMA tiles), 128-byte stages, A and B double-buffered. (A
     // triple-buffered, running a stage further ahead than B in the 32 KiB of LDS left over, measured
     // 1030-1034 against 1300-1307 TFLOP/s on one box: correct, and slower.)
     if (choice == 4128) return gemm4_launch_cfg<KIND, OUT, 2>(s, d, c, a, b, scale, acc_out);
   }
+  if (choice == 32)
+    return gemm_launch_cfg<KIND, OUT, 32, 64, 1, 2, 4>(s, d, c, a, b, scale, acc_out,
+                                                       splits_of(t64, d.K * MfmaT<KIND>::EB, 32), &ws);
   if (choice == 64)
     return gemm_launch_cfg<KIND, OUT, 64, 64, 2, 2, 4>(s, d, c, a, b, scale, acc_out,
-                                                       splits_of(t64, d.K * MfmaT<KIND>::EB), &ws);
+                                                       splits_of(t64, d.K * MfmaT<KIND>::EB, 64), &ws);
   if (choice == 1284) return gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 4>(s, d, c, a, b, scale, acc_out);
   if (choice == 128) return gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 2>(s, d, c, a, b, scale, acc_out);
   return gemm_launch_cfg<KIND, OUT, 256, 256, 2, 4, 2>(s, d, c, a, b, scale, acc_out);
