@@ -441,9 +441,10 @@ void launch_rmsnorm_softmax(hipStream_t s, uint16_t* out, const uint16_t* x, con
   // at 4 MiB 5.3 against 4.5).
   const bool aligned = (((uintptr_t)x | (uintptr_t)out | (uintptr_t)gain) & 15) == 0;
   const bool stream = rows * cols * 2 >= (10ll << 20);
+  const int64_t row_threads = cols <= 1024 ? 64 : cols <= 4096 ? 256 : cols <= 8192 ? 512 : 1024;  // at most
   if (aligned && cols == 4096 && rows >= 6144) {
     rs_dma_launch<8>(s, out, x, gain, rows, eps);
-  } else if (cols <= 32768 && rows < (1ll << 31)) {
+  } else if (cols <= 32768 && rows * row_threads < (1ll << 32)) {  // a launch's threads fit 32 bits
     if (cols <= 512)
       rs_row_launch<8, 1>(s, out, x, gain, rows, cols, eps, stream);
     else if (cols <= 1024)

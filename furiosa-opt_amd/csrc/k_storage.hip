@@ -345,7 +345,7 @@ void relayout_t(hipStream_t s, void* dst, const void* src, int64_t dst_base, int
   if (w.n >= 1 && w.stride[0][0] == 1 && count % w.size[0] == 0 && w.live[0] * sizeof(T) >= 8) {
     const int64_t bytes = w.live[0] * (int64_t)sizeof(T), runs = count / w.size[0];
     const int wb = bytes >= 16 ? 16 : 8;
-    if (runs * ((bytes + wb - 1) / wb) < (1ll << 31)) {
+    if (bytes < (1ll << 31) && runs * ((bytes + wb - 1) / wb) < (1ll << 31)) {  // 32-bit piece offsets
       uint8_t* d = (uint8_t*)dst + dst_base * (int64_t)sizeof(T);
       const uint8_t* r = (const uint8_t*)src + src_base * (int64_t)sizeof(T);
       return wb == 16 ? runs_launch<16>(s, d, r, sizeof(T), runs, w) : runs_launch<8>(s, d, r, sizeof(T), runs, w);
