@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # units at and past the powers of two, more units than a block stages at once, the one-row forms' edges.
 SHAPES = [(1, 31, 100, 2), (3, 129, 16, 64), (2, 100, 1024, 63), (5, 33, 513, 17), (256, 72, 130, 9), (257, 72, 130, 9),
           (513, 65, 33, 16), (1025, 40, 64, 10), (2049, 24, 128, 5), (2050, 33, 257, 10), (2100, 1000, 512, 64),
-          (300, 1024, 20, 33), (1, 4000, 1024, 64), (7, 100, 28, 3)]
+          (300, 1024, 20, 33), (512, 72, 64, 9), (513, 72, 64, 9), (257, 72, 65, 9), (1, 4000, 1024, 64), (7, 100, 28, 3)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
