@@ -9,16 +9,18 @@
 // reference's bf16 rule (float/bf16.rs:16-40: a subnormal reads as a signed zero); the products
 // and sums themselves are IEEE f32, subnormal results included. The parallelism is across cells,
 // and the chain of K dependent adds per cell bounds a small GEMV, HBM a large one. Two kernels:
-//   * k_gemv_fold (K <= 4096): a block of seven waves owns 64 cells. Waves 1-6 stream the 64 weight
+//   * k_gemv_fold (K <= 4096): a block of four waves owns 16 or 32 cells. Waves 1-3 stream the weight
 //     rows from HBM (16-byte loads, four stages in flight) and write the exact f32 products of each
 //     96-element stage to LDS; wave 0 folds the previous stage's products, one cell per lane, so its
-//     instruction stream is one LDS read per four adds. (Three producer waves left the fold waiting
-//     on them; six bring a stage close to the folder's own chain of dependent adds.) The producer waves run with subnormal inputs
+//     instruction stream is one LDS read per four adds. (A 64-cell block needed six producer waves to
+//     keep up with the folder, and their LDS traffic slowed it.) The producer waves run with subnormal inputs
 //     flushed and subnormal results kept (the MODE register is per wave): the reference's widen of
 //     a subnormal weight to zero, then an IEEE product. The folding wave keeps full IEEE behaviour.
 //   * k_gemv_bf16 (any K): R cells per block, the rows staged through LDS by all waves and folded by
 //     the first R lanes of wave 0, widening each weight on the fly.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "runtime.hpp"
 
@@ -124,15 +126,12 @@ __global__ void __launch_bounds__(kGemvThreads) k_gemv_bf16(Out* __restrict__ ou
   if (folder && n0 + t < N) out[(n0 + t) * ldo] = narrow_out<Out>(acc);
 }
 
-constexpr int kFoldR = 64;                          // cells per block: one per lane of wave 0
 constexpr int kFoldKC = 96;                         // k elements per stage
 constexpr int kFoldCPR = kFoldKC / 8;               // 16-byte chunks per row per stage
-constexpr int kFoldProducers = 384;                 // threads of waves 1-6
-constexpr int kFoldPer = kFoldR * kFoldCPR / kFoldProducers;  // chunks per producer per stage (4)
+constexpr int kFoldProducers = 192;                 // threads of waves 1-3
 constexpr int kFoldPS = kFoldKC + 4;  // product row stride in floats: 16 lanes' b128 reads cover 64 banks once
 constexpr int kFoldMaxK = 4096;       // x is staged whole in LDS
 constexpr int kFoldDepth = 4;         // stages of weight loads in flight per producer
-static_assert(kFoldR * kFoldCPR % kFoldProducers == 0, "producer chunks must divide evenly");
 // s_waitcnt lgkmcnt(0) with vmcnt and expcnt left alone: LDS traffic done, global loads still in flight.
 constexpr int kWaitLds = 15 | (7 << 4) | (0 << 8) | (3 << 14);
 // MODE.FP_DENORM single-precision field (bits 5:4) = 2: flush subnormal inputs, keep subnormal results.
@@ -141,16 +140,19 @@ constexpr int kDenormFlushIn = 2;
 
 // XF32: x is f32 data standing for the widen of its deferred bf16 narrow (the runtime's deferred
 // casts); each element is rounded to bf16 by the narrow's rule and widened as it is staged.
-template <typename Out, bool XF32>
+// R: cells per block, one per lane of wave 0.
+template <int R, typename Out, bool XF32>
 __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restrict__ out, const void* __restrict__ x,
                                                    const uint16_t* __restrict__ w, int64_t N, int K, int64_t ldw,
                                                    int64_t ldo) {
-  __shared__ __attribute__((aligned(16))) float P[2][kFoldR * kFoldPS];
+  constexpr int kPer = R * kFoldCPR / kFoldProducers;  // chunks per producer per stage
+  static_assert(R * kFoldCPR % kFoldProducers == 0, "producer chunks must divide evenly");
+  __shared__ __attribute__((aligned(16))) float P[2][R * kFoldPS];
   __shared__ __attribute__((aligned(16))) float xs[kFoldMaxK];
   const int t = threadIdx.x;
   const bool folder = __builtin_amdgcn_readfirstlane(t >> 6) == 0;  // wave 0 (uniform per wave)
   const int p = t - 64;
-  const int64_t n0 = (int64_t)blockIdx.x * kFoldR;
+  const int64_t n0 = (int64_t)blockIdx.x * R;
   const int stages = (K + kFoldKC - 1) / kFoldKC;
   const int xchunks = K / 8;
 
@@ -160,29 +162,29 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
   // A producer's chunks sit at fixed (row, column) places of every stage: their row pointers,
   // columns and product offsets are computed once.
   // The producers are a whole number of rows, so all of a producer's chunks share a column, and one read
-  // of x's eight values serves them (a read per chunk kept the LDS pipe as busy as the fold: K = 1024 7.0
-  // -> 6.3 us, 3072 15.7 -> 14.2, the 155,648-row head 62 -> 60).
+  // of x's eight values serves them (with 64 cells a block, a read per chunk kept the LDS pipe as busy
+  // as the fold: K = 1024 7.0 -> 6.3 us, 3072 15.7 -> 14.2, the 155,648-row head 62 -> 60).
   static_assert(kFoldProducers % kFoldCPR == 0, "a producer's chunks share a column");
-  const uint16_t* wrow[kFoldPer];
-  int poff[kFoldPer];
+  const uint16_t* wrow[kPer];
+  int poff[kPer];
   const int pcol = (p % kFoldCPR) * 8;
 #pragma unroll
-  for (int u = 0; u < kFoldPer; ++u) {
+  for (int u = 0; u < kPer; ++u) {
     const int row = (p + u * kFoldProducers) / kFoldCPR;
     poff[u] = row * kFoldPS + pcol;
     wrow[u] = w + min(n0 + row, N - 1) * ldw;
   }
-  uint4 reg[kFoldDepth][kFoldPer];
-  auto load = [&](int s, uint4 (&r)[kFoldPer]) {
+  uint4 reg[kFoldDepth][kPer];
+  auto load = [&](int s, uint4 (&r)[kPer]) {
     const int k0 = s * kFoldKC;
     const bool full = k0 + kFoldKC <= K;  // uniform: no chunk of the stage reaches K
     const int k = k0 + pcol, kk = full || k < K ? k : K - 8;
 #pragma unroll
-    for (int u = 0; u < kFoldPer; ++u) r[u] = *(const uint4*)(wrow[u] + kk);
+    for (int u = 0; u < kPer; ++u) r[u] = *(const uint4*)(wrow[u] + kk);
   };
   if (!folder) {
     __builtin_amdgcn_s_setreg(kModeDenormF32, kDenormFlushIn);
-    constexpr int kXPer = kFoldMaxK / 8 / kFoldProducers + 1;  // x chunks per producer (3)
+    constexpr int kXPer = (kFoldMaxK / 8 + kFoldProducers - 1) / kFoldProducers;  // x chunks per producer (3)
     uint4 xv[kXPer][XF32 ? 2 : 1];
 #pragma unroll
     for (int u = 0; u < kXPer; ++u) {
@@ -239,12 +241,12 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
         const int s = r * kFoldDepth + j;
         // The products of stage s into P[s & 1]; FULL (a constant at each inlined use) when every
         // chunk of the stage lies below K, else chunks past K write +0.
-        auto produce = [&](int s, const uint4 (&r)[kFoldPer], bool FULL) __attribute__((always_inline)) {
+        auto produce = [&](int s, const uint4 (&r)[kPer], bool FULL) __attribute__((always_inline)) {
           float* dst = P[s & 1];
           const int k = s * kFoldKC + pcol, kk = FULL || k < K ? k : K - 8;
           const float4 xa = *(const float4*)&xs[kk], xb = *(const float4*)&xs[kk + 4];
 #pragma unroll
-          for (int u = 0; u < kFoldPer; ++u) {
+          for (int u = 0; u < kPer; ++u) {
             const uint4 v = r[u];
             float4 a = make_float4(__fmul_rn(xa.x, bf16_lo(v.x)), __fmul_rn(xa.y, bf16_hi(v.x)),
                                    __fmul_rn(xa.z, bf16_lo(v.y)), __fmul_rn(xa.w, bf16_hi(v.y)));
@@ -268,7 +270,7 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
 #pragma unroll
       for (int j = 0; j < kFoldDepth; ++j) {
         const int s = r * kFoldDepth + j;
-        if (s >= 1 && s <= stages) {
+        if (s >= 1 && s <= stages && t < R) {
           // Products past K are +0, which leave the sum unchanged. The stage's row is read whole
           // before the adds (all reads in flight at once, not one read's latency per four adds).
           const float* row = &P[(s - 1) & 1][t * kFoldPS];
@@ -288,19 +290,23 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
       }
     }
   }
-  if (folder && n0 + t < N) out[(n0 + t) * ldo] = narrow_out<Out>(acc);
+  if (t < R && n0 + t < N) out[(n0 + t) * ldo] = narrow_out<Out>(acc);
 }
 
-template <typename Out>
+template <int R, typename Out>
 void gemv_fold(hipStream_t s, Out* out, const void* x, bool x_f32, const uint16_t* w, int64_t N, int64_t K,
                int64_t ldw, int64_t ldo) {
-  const int64_t blocks = (N + kFoldR - 1) / kFoldR;
-  if (x_f32)
-    hipLaunchKernelGGL((k_gemv_fold<Out, true>), dim3((unsigned)blocks), dim3(64 + kFoldProducers), 0, s, out, x, w,
-                       N, (int)K, ldw, ldo);
-  else
-    hipLaunchKernelGGL((k_gemv_fold<Out, false>), dim3((unsigned)blocks), dim3(64 + kFoldProducers), 0, s, out, x, w,
-                       N, (int)K, ldw, ldo);
+  constexpr int64_t kLaunchRows = (int64_t)R << 23;  // a launch's threads fit 32 bits
+  for (int64_t n = 0; n < N; n += kLaunchRows) {
+    const int64_t rows = std::min(N - n, kLaunchRows);
+    const dim3 grid((unsigned)((rows + R - 1) / R)), block(64 + kFoldProducers);
+    if (x_f32)
+      hipLaunchKernelGGL((k_gemv_fold<R, Out, true>), grid, block, 0, s, out + n * ldo, x, w + n * ldw, rows, (int)K,
+                         ldw, ldo);
+    else
+      hipLaunchKernelGGL((k_gemv_fold<R, Out, false>), grid, block, 0, s, out + n * ldo, x, w + n * ldw, rows, (int)K,
+                         ldw, ldo);
+  }
   FO_HIP(hipGetLastError());
 }
 
@@ -334,10 +340,20 @@ void launch_gemv(hipStream_t s, void* out, const void* x, const void* w, fo_dtyp
   require(!x_f32 || gemv_takes_f32_x(K), "gemv: an f32 x through its bf16 narrow takes K <= 4096");
   const uint16_t *xp = (const uint16_t*)x, *wp = (const uint16_t*)w;
   if (K <= kFoldMaxK) {
-    if (out_t == FO_F32)
-      gemv_fold<float>(s, (float*)out, x, x_f32, wp, N, K, ldw, ldo);
+    // 16 cells a block while the 256 CUs each take at most one block, else 32: fewer cells leave the LDS
+    // pipe to the fold (16 rows of reads and products a stage, not 64) and spread a small N over more CUs.
+    // Kernel alone in a recorded graph, N x K, us, 64 cells and six producer waves / 32 and three / 16 and
+    // three: 1024 x 1024 6.45 / 5.82 / 5.63; 3072 x 1024 6.58 / 5.90 / 5.73; 1024 x 3072 14.6 / 12.4 / 12.2;
+    // 155648 x 1024 60.9 / 59.1 / 70.6. (32 cells and six waves: 5.94, 6.08, 13.4, 70.6.)
+    const bool few = N <= 16 * 256;
+    if (out_t == FO_F32 && few)
+      gemv_fold<16>(s, (float*)out, x, x_f32, wp, N, K, ldw, ldo);
+    else if (out_t == FO_F32)
+      gemv_fold<32>(s, (float*)out, x, x_f32, wp, N, K, ldw, ldo);
+    else if (few)
+      gemv_fold<16>(s, (uint16_t*)out, x, x_f32, wp, N, K, ldw, ldo);
     else
-      gemv_fold<uint16_t>(s, (uint16_t*)out, x, x_f32, wp, N, K, ldw, ldo);
+      gemv_fold<32>(s, (uint16_t*)out, x, x_f32, wp, N, K, ldw, ldo);
     return;
   }
   // Rows per block: 64 where that still gives 512 blocks, else fewer so a small N spreads out.
