@@ -59,6 +59,12 @@ constexpr int kBN = 64;   // keys per block
 constexpr float kEps = 6.25e-8f;  // attention.rs:13
 constexpr float kL2E = 1.4426950408889634f;
 constexpr float kTau = 5.545177444479562f;  // 8 ln 2: p = exp(s - m_run) <= 2^8 between rescales
+// The running max starts below every bf16 logit whose product with log2(e) is finite (the lowest is
+// -2.353e38), and that product is finite for it too: a -inf logit (q.k overflowed) has p = 0 from the
+// first block on. A row's p sums to 0 only where no visible logit is above kLow; its output is NaN, as
+// the softmax of nothing but -inf is.
+constexpr float kLow = -2.358e38f;
+constexpr int kNan2 = 0x7fc07fc0;  // two bf16 NaN
 
 __device__ __forceinline__ f32x16_t mma(const i32x4_t& a, const i32x4_t& b, const f32x16_t& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0,
@@ -172,9 +178,8 @@ __device__ __forceinline__ void attn_step(const uint8_t* __restrict__ sK, const 
   // Online softmax step with a lazy reference max: O and the sum are rescaled only when some
   // lane's block max exceeds its reference max by more than kTau, so p = exp(s - m_run) stays
   // <= e^kTau = 256 and most blocks skip the rescale of the 64 O registers. The ratio O / sum
-  // does not depend on the reference (every p of a row shares it). Every query of a processed
-  // block sees key 0 of the first block, so the first block always rescales (alpha = 0 there,
-  // m_run = -inf) and m_run is finite from then on.
+  // does not depend on the reference (every p of a row shares it). The first block with a logit above
+  // kLow always rescales (alpha = 0 there), and m_run is that row's own from then on.
   if (bmax > m_run + kTau) {  // per lane: skipped as a whole when no lane of the wave needs it
     const float alpha = __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, kL2E, -bmax * kL2E));
     m_run = bmax;
@@ -347,8 +352,8 @@ __global__ void __launch_bounds__(kNT, 2 * 4 / kWaves) k_attn_fwd(uint16_t* __re
   for (int t = 0; t < C::DT; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
-  float m_run = -INFINITY, l_part = 0.f;
-  if (row_max && myq < seq) m_run = row_max[head * (int64_t)seq + myq];
+  float m_run = GIVEN ? -INFINITY : kLow, l_part = 0.f;
+  if (GIVEN && myq < seq) m_run = row_max[head * (int64_t)seq + myq];
 
   // Buffers: K(j) and V(j) live in buffer j % 2. Step j reads them, and after it writes K(j+1)
   // and V(j+1) (loaded during the step) into buffer (j+1) % 2, last read by step j-1 before the
@@ -389,13 +394,14 @@ __global__ void __launch_bounds__(kNT, 2 * 4 / kWaves) k_attn_fwd(uint16_t* __re
   }
 
   // out[myq][d] = bf16( bf16(o) / (l + EPS) ); lane holds d = 32t + 8*(r/4) + 4g + r%4. The
-  // quotient is correctly rounded (the divisor is normal: l >= 1 with the running max, l + EPS >=
-  // EPS with a given one; |o| <= l max|v| keeps the quotient finite); both narrows are the
-  // hardware's round-to-nearest-even (finite inputs give finite, normal-or-zero o).
+  // quotient is correctly rounded (the divisor is normal: l >= 1 with the running max unless the row is
+  // `none` below, l + EPS >= EPS with a given one; |o| <= l max|v| keeps the quotient finite); both narrows
+  // are the hardware's round-to-nearest-even (finite inputs give finite, normal-or-zero o).
   const LanePair lp = half_pair(l_part);
   const float l_run = lp.lo + lp.hi;
   // Every lane computes (a query past the end sees every key, so its l >= 1 too); lanes l and
   // l + 32 hold the same query row, so the regrouped 16-byte stores share one condition.
+  const bool none = !GIVEN && l_run == 0.f;
   const float denom = l_run + kEps;
   const float rinv = __fdiv_rn(1.0f, denom);
   uint16_t* orow = out + head * (int64_t)seq * D + (int64_t)myq * D;
@@ -411,7 +417,8 @@ __global__ void __launch_bounds__(kNT, 2 * 4 / kWaves) k_attn_fwd(uint16_t* __re
           const int blk = bp + d;
           wv[d][e] = (int)normalized_pair(o[t][blk * 4 + 2 * e], o[t][blk * 4 + 2 * e + 1], denom, rinv);
         }
-      const i32x4_t q4 = regroup8(wv[0], wv[1]);
+      i32x4_t q4 = regroup8(wv[0], wv[1]);
+      if (none) q4 = i32x4_t{kNan2, kNan2, kNan2, kNan2};
       if (myq < seq) *(i32x4_t*)(orow + t * 32 + 8 * bp + 8 * g) = q4;
     }
 }
@@ -425,10 +432,8 @@ __global__ void __launch_bounds__(kNT, 2 * 4 / kWaves) k_attn_fwd(uint16_t* __re
 // the online softmax's rescale, one 32-row tile of O per wave. Bound by latency: a step of the 2 x 4 form
 // takes 3.4 us (loads, LDS stores, barrier, S, softmax and PV in turn: the four blocks fill the LDS, so
 // nothing is double-buffered), of the 4 x 2 form 2.3 us, against 1.8 us for one block of the 256-query form.
-// Four waves of one query group by four key groups measured no faster (600 keys: 15.4 us). The running max starts at a finite
-// value below any logit (kLow), so a wave that has seen no visible key yet holds (kLow, 0, 0) and
-// weighs nothing in the combine.
-constexpr float kLow = -2.3e38f;  // kLow * log2(e) is still finite
+// Four waves of one query group by four key groups measured no faster (600 keys: 15.4 us). The running max starts at
+// kLow, so a wave that has seen no visible key yet holds (kLow, 0, 0) and weighs nothing in the combine.
 
 template <int D, int QG, int KG>
 struct SplitCfg {
@@ -580,6 +585,7 @@ __global__ void __launch_bounds__(64 * QG * KG, QG * KG <= 4 ? 1 : 2) k_attn_spl
     f[i] = __builtin_amdgcn_exp2f((sml[((i * QG + qg) * 2) * 64 + lane] - m) * kL2E);
     l += f[i] * sml[((i * QG + qg) * 2 + 1) * 64 + lane];
   }
+  const bool none = l == 0.f;
   const float denom = l + kEps;
   const float rinv = __fdiv_rn(1.0f, denom);
   uint16_t* orow = out + at + (int64_t)myq * D;
@@ -606,7 +612,8 @@ __global__ void __launch_bounds__(64 * QG * KG, QG * KG <= 4 ? 1 : 2) k_attn_spl
       for (int d = 0; d < 2; ++d)
 #pragma unroll
         for (int e = 0; e < 2; ++e) wv[d][e] = (int)normalized_pair(s[(bp + d) * 4 + 2 * e], s[(bp + d) * 4 + 2 * e + 1], denom, rinv);
-      const i32x4_t q4 = regroup8(wv[0], wv[1]);
+      i32x4_t q4 = regroup8(wv[0], wv[1]);
+      if (none) q4 = i32x4_t{kNan2, kNan2, kNan2, kNan2};
       if (myq < seq) *(i32x4_t*)(orow + t * 32 + 8 * bp + 8 * g) = q4;
     }
   }
