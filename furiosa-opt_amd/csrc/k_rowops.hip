@@ -91,6 +91,13 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
+// With gains below this, and a finite sum of squares, |y_i| <= sqrt(cols) * max|g| < 2^7.5 * 2^21 at the
+// 32768 columns the kernels take (|x_i| <= sqrt(ss), r >= sqrt(ss / cols)). exp2 of the fused
+// y * log2(e) - RN(max * log2(e)) leaves the rounding of the product, up to 2^-24 of it, as a common
+// factor of the row: below 2^6 in the exponent then, which the sum divides out; past it the row's
+// exponentials overflow or all vanish.
+constexpr float kGainMax = 0x1p21f;
+
 // The exact per-element path (reference rules at every rounding point), for rows holding a
 // non-finite value. Reads the row again from global memory.
 __device__ void row_exact(uint16_t* __restrict__ orow, const uint16_t* __restrict__ xr,
@@ -163,16 +170,14 @@ __global__ void __launch_bounds__(64 * kDmaWaves) k_rmsnorm_softmax_dma(uint16_t
   int64_t row = __builtin_amdgcn_readfirstlane((int)wave);
   if (row < rows) fetch(row);  // overlaps the gain staging below
   // The gain row is shared by every row: widen it once per block into LDS (reference widen rule),
-  // and note whether it holds a non-finite value or a magnitude of 2^120 or more (below that no y
-  // can overflow once the row's sum of squares is finite: |x_i| <= sqrt(ss) and r >= sqrt(ss / cols)
-  // give |y_i| <= sqrt(cols) * max|g| < 2^7 * 2^120).
+  // and note whether it holds a non-finite value or a magnitude of kGainMax or more.
   // Each thread checks the gain values it stages; one workgroup reduction combines the checks (it
   // also orders the staging before every wave's reads).
   int bad_local = 0;
   for (int i = threadIdx.x; i < cols; i += blockDim.x) {
     const float gv = bf16_to_f32(gain[i]);
     sg[i] = gv;
-    bad_local |= !(__builtin_fabsf(gv) < 0x1p120f);
+    bad_local |= !(__builtin_fabsf(gv) < kGainMax);
   }
   __syncthreads();
   const bool gain_bad = __syncthreads_or(bad_local) != 0;
@@ -332,12 +337,12 @@ __global__ void __launch_bounds__(W < 4 ? 256 : 64 * W) k_rmsnorm_softmax_row(ui
   }
   float y[P];
   float ss = 0.f;
-  bool bad = false;
+  bool bad = false;  // a gain of kGainMax or more
 #pragma unroll
   for (int i = 0; i < P; ++i) {
     y[i] = bits_f32((uint32_t)xv[i / 8][i % 8] << 16);
     ss = __builtin_fmaf(y[i], y[i], ss);  // a bf16 square is exact in f32
-    bad |= !(__builtin_fabsf(bits_f32((uint32_t)gv[i / 8][i % 8] << 16)) < 0x1p120f);
+    bad |= !(__builtin_fabsf(bits_f32((uint32_t)gv[i / 8][i % 8] << 16)) < kGainMax);
   }
   ss = combine(0, bad ? INFINITY : ss, false);
   const bool exact = !__builtin_isfinite(ss);  // uniform over the row's waves

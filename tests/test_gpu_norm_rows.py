@@ -52,3 +52,25 @@ def test_rmsnorm_softmax_rows_nonfinite(rt, cols):
         if not huge:
             bound = rmsnorm_bound(x.ravel(), g, rows, cols, 1e-6)
             close_chain(got[fin], want[fin], frac_beyond=1e-4, hard=bound[fin])
+
+
+@pytest.mark.parametrize("shape", [(3, 512), (3, 999), (6144, 4096), (3, 32000), (3, 32768)], ids=lambda s: "x".join(map(str, s)))
+def test_rmsnorm_softmax_rows_large_gain(rt, shape):
+    """One nonzero value a row against gains up to where y overflows: y is the largest a finite row gives,
+    sqrt(cols) times the gain, and its softmax is one there and zero elsewhere."""
+    rows, cols = shape
+    x = np.zeros((rows, cols), np.float32)
+    x[:, 17] = 1.0
+    x[1, 17], x[1, cols - 1], x[2, 17] = 0.0, 3.0, -1.0
+    x = emu.f32_to_bf16(x.ravel())
+    for gain in (2.0 ** 20, 2.0 ** 21, 2.0 ** 24 * 1.5, 2.0 ** 60, 2.0 ** 119 * 1.9921875, 2.0 ** 120):
+        g = emu.f32_to_bf16(np.full(cols, gain, np.float32))
+        want = emu.bf16_to_f32(emu.rmsnorm_softmax(x[:3 * cols], g, 3, cols, 1e-6)).reshape(3, cols)
+        assert want[0, 17] == 1.0 and want[1, cols - 1] == 1.0 and want[2, 17] == 0.0
+        out = rt.alloc(rows * cols * 2)
+        print(f"rmsnorm_softmax large gain {shape} {gain}", flush=True)
+        rt.rmsnorm_softmax(out, rt.upload(x), rt.upload(g), rows, cols, 1e-6)
+        got = emu.bf16_to_f32(out.read(np.uint16)).reshape(rows, cols)
+        assert np.array_equal(got[:2], want[:2]) and np.all(got[3:] == want[0])
+        # the third row's equal weights are 1 / (cols - 1) each, within a rounding to bf16 either way
+        assert np.all(np.abs(got[2] - want[2]) <= 2.0 ** -7 * want[2])
