@@ -19,7 +19,8 @@
 // subnormal reads as zero in every later op), a subnormal result flushes before the narrow, and
 // the narrow is the hardware round-to-nearest-even v_cvt_pk_bf16_f32. The one case left is a
 // non-finite value (NaN payloads and inf - inf), which the reference canonicalises: a row whose
-// sum of squares, gain or y is non-finite is recomputed by the exact per-element path.
+// sum of squares is non-finite, whose mean square is not positive (a division by zero) or whose gain
+// reaches kGainMax is computed by the exact per-element path.
 //   * (x*g)/r is the correctly rounded quotient q' = RN(q + e*y), q = RN(a*y), e = a - q*r (exact,
 //     one FMA), y = RN(1/r) (Markstein's correction, exact for normal operands and results);
 //   * exp and the final division feed only the output's bf16 narrow, so they use the hardware exp2
@@ -205,12 +206,12 @@ __global__ void __launch_bounds__(64 * kDmaWaves) k_rmsnorm_softmax_dma(uint16_t
     }
     const float ss = wave_sum(ss0 + ss1);
     uint16_t* orow = out + row * cols;
-    if (!__builtin_isfinite(ss) || gain_bad) {
+    const float ms = __fadd_rn(__fdiv_rn(ss, cols_f), eps);  // fp_div, then clip Add eps
+    if (!__builtin_isfinite(ss) || !(ms > 0.f) || gain_bad) {
       row_exact(orow, x + row * cols, gain, cols, eps, lane);
       __builtin_amdgcn_s_waitcnt(waitcnt_vm0);
       continue;
     }
-    const float ms = __fadd_rn(__fdiv_rn(ss, cols_f), eps);  // fp_div, then clip Add eps
     const float r = sqrt_rn(ms);                              // FpUnaryOp::Sqrt
     const float rinv = __fdiv_rn(1.0f, r);
     // y = bf16((x * g) / r), kept packed; row max on the f32 values
@@ -345,8 +346,8 @@ __global__ void __launch_bounds__(W < 4 ? 256 : 64 * W) k_rmsnorm_softmax_row(ui
     bad |= !(__builtin_fabsf(bits_f32((uint32_t)gv[i / 8][i % 8] << 16)) < kGainMax);
   }
   ss = combine(0, bad ? INFINITY : ss, false);
-  const bool exact = !__builtin_isfinite(ss);  // uniform over the row's waves
   const float ms = __fadd_rn(__fdiv_rn(ss, (float)cols), eps);  // fp_div, then clip Add eps
+  const bool exact = !__builtin_isfinite(ss) || !(ms > 0.f);  // uniform over the row's waves
   const float r = sqrt_rn(ms);                                    // FpUnaryOp::Sqrt
   const float rinv = __fdiv_rn(1.0f, r);
   float mx = -INFINITY;

@@ -74,3 +74,22 @@ def test_rmsnorm_softmax_rows_large_gain(rt, shape):
         assert np.array_equal(got[:2], want[:2]) and np.all(got[3:] == want[0])
         # the third row's equal weights are 1 / (cols - 1) each, within a rounding to bf16 either way
         assert np.all(np.abs(got[2] - want[2]) <= 2.0 ** -7 * want[2])
+
+
+@pytest.mark.parametrize("shape", [(3, 64), (3, 500), (3, 1024), (3, 5000), (2, 20000), (6144, 4096)], ids=lambda s: "x".join(map(str, s)))
+def test_rmsnorm_softmax_rows_no_mean_square(rt, shape):
+    """Without an eps, a row of zeros and a row whose squares all flush to zero divide by zero: their outputs
+    are the reference's NaN, bit for bit."""
+    rows, cols = shape
+    x = np.full((rows, cols), 0x3F80, np.uint16)
+    x[0], x[rows - 1] = 0, 0x8080  # zeros; the smallest normal bf16, negative
+    x[rows - 1, 0] = 0x0080
+    g = emu.f32_to_bf16(np.ones(cols, np.float32))
+    want = emu.rmsnorm_softmax(x[[0, 1, rows - 1]].ravel(), g, 3, cols, 0.0).reshape(3, cols)
+    out = rt.alloc(rows * cols * 2)
+    print(f"rmsnorm_softmax no mean square {rows}x{cols}", flush=True)
+    rt.rmsnorm_softmax(out, rt.upload(x.ravel()), rt.upload(g), rows, cols, 0.0)
+    got = out.read(np.uint16).reshape(rows, cols)
+    assert np.all(want[[0, 2]] == 0x7FC0) and np.array_equal(got[[0, rows - 1]], want[[0, 2]])
+    if rows > 2:
+        assert np.array_equal(got[1], want[1])
