@@ -20,8 +20,7 @@
 //     the first R lanes of wave 0, widening each weight on the fly.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
+#include "launch_rules.hpp"
 #include "runtime.hpp"
 
 namespace fo {
@@ -296,9 +295,8 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
 template <int R, typename Out>
 void gemv_fold(hipStream_t s, Out* out, const void* x, bool x_f32, const uint16_t* w, int64_t N, int64_t K,
                int64_t ldw, int64_t ldo) {
-  constexpr int64_t kLaunchRows = (int64_t)R << 23;  // a launch's threads fit 32 bits
-  for (int64_t n = 0; n < N; n += kLaunchRows) {
-    const int64_t rows = std::min(N - n, kLaunchRows);
+  static_assert((64 + kFoldProducers) % R == 0, "threads a row");
+  for_row_pieces(N, (64 + kFoldProducers) / R, [&](int64_t n, int64_t rows) {
     const dim3 grid((unsigned)((rows + R - 1) / R)), block(64 + kFoldProducers);
     if (x_f32)
       hipLaunchKernelGGL((k_gemv_fold<R, Out, true>), grid, block, 0, s, out + n * ldo, x, w + n * ldw, rows, (int)K,
@@ -306,7 +304,7 @@ void gemv_fold(hipStream_t s, Out* out, const void* x, bool x_f32, const uint16_
     else
       hipLaunchKernelGGL((k_gemv_fold<R, Out, false>), grid, block, 0, s, out + n * ldo, x, w + n * ldw, rows, (int)K,
                          ldw, ldo);
-  }
+  });
   FO_HIP(hipGetLastError());
 }
 

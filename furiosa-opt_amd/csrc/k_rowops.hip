@@ -28,6 +28,7 @@
 //   * the row max is taken on f32 y: rounding to nearest is monotone, so bf16(max y) = max bf16(y).
 #include <hip/hip_runtime.h>
 
+#include "launch_rules.hpp"
 #include "runtime.hpp"
 
 namespace fo {
@@ -411,11 +412,15 @@ template <int P, int W>
 void rs_row_launch(hipStream_t s, uint16_t* out, const uint16_t* x, const uint16_t* g, int64_t rows, int64_t cols,
                    float eps, bool stream) {
   constexpr int R = W < 4 ? 4 / W : 1;
-  const dim3 grid((unsigned)((rows + R - 1) / R)), block(W < 4 ? 256 : 64 * W);
-  if (stream)
-    hipLaunchKernelGGL((k_rmsnorm_softmax_row<P, W, true>), grid, block, 0, s, out, x, g, rows, (int)cols, eps);
-  else
-    hipLaunchKernelGGL((k_rmsnorm_softmax_row<P, W, false>), grid, block, 0, s, out, x, g, rows, (int)cols, eps);
+  for_row_pieces(rows, 64 * W, [&](int64_t first, int64_t n) {
+    const dim3 grid((unsigned)((n + R - 1) / R)), block(W < 4 ? 256 : 64 * W);
+    uint16_t* o = out + first * cols;
+    const uint16_t* in = x + first * cols;
+    if (stream)
+      hipLaunchKernelGGL((k_rmsnorm_softmax_row<P, W, true>), grid, block, 0, s, o, in, g, n, (int)cols, eps);
+    else
+      hipLaunchKernelGGL((k_rmsnorm_softmax_row<P, W, false>), grid, block, 0, s, o, in, g, n, (int)cols, eps);
+  });
 }
 
 // Rows past 32768 columns: the exact per-element path, one wave per row.
@@ -447,10 +452,9 @@ void launch_rmsnorm_softmax(hipStream_t s, uint16_t* out, const uint16_t* x, con
   // at 4 MiB 5.3 against 4.5).
   const bool aligned = (((uintptr_t)x | (uintptr_t)out | (uintptr_t)gain) & 15) == 0;
   const bool stream = rows * cols * 2 >= (10ll << 20);
-  const int64_t row_threads = cols <= 1024 ? 64 : cols <= 4096 ? 256 : cols <= 8192 ? 512 : 1024;  // at most
   if (aligned && cols == 4096 && rows >= 6144) {
     rs_dma_launch<8>(s, out, x, gain, rows, eps);
-  } else if (cols <= 32768 && rows * row_threads < (1ll << 32)) {  // a launch's threads fit 32 bits
+  } else if (cols <= 32768) {
     if (cols <= 512)
       rs_row_launch<8, 1>(s, out, x, gain, rows, cols, eps, stream);
     else if (cols <= 1024)
@@ -470,8 +474,10 @@ void launch_rmsnorm_softmax(hipStream_t s, uint16_t* out, const uint16_t* x, con
     else
       rs_row_launch<32, 16>(s, out, x, gain, rows, cols, eps, stream);
   } else {
-    hipLaunchKernelGGL(k_rmsnorm_softmax_any, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, out, x, gain, rows,
-                       cols, eps);
+    for_row_pieces(rows, 64, [&](int64_t first, int64_t n) {
+      hipLaunchKernelGGL(k_rmsnorm_softmax_any, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, out + first * cols,
+                         x + first * cols, gain, n, cols, eps);
+    });
   }
   FO_HIP(hipGetLastError());
 }

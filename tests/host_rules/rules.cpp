@@ -1,0 +1,25 @@
+// Prints what the launch rules choose: one question a line on stdin, one answer a line on stdout.
+#include <cstdio>
+#include <iostream>
+#include <sstream>
+#include <string>
+
+#include "launch_rules.hpp"
+
+int main() {
+  std::string line;
+  while (std::getline(std::cin, line)) {
+    std::istringstream in(line);
+    std::string rule;
+    in >> rule;
+    if (rule == "pieces") {
+      int64_t rows, threads;
+      in >> rows >> threads;
+      fo::for_row_pieces(rows, threads, [](int64_t first, int64_t count) { std::printf("%lld+%lld ", (long long)first, (long long)count); });
+      std::printf("\n");
+    } else {
+      return 1;
+    }
+  }
+  return 0;
+}

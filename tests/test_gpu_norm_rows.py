@@ -93,3 +93,20 @@ def test_rmsnorm_softmax_rows_no_mean_square(rt, shape):
     assert np.all(want[[0, 2]] == 0x7FC0) and np.array_equal(got[[0, rows - 1]], want[[0, 2]])
     if rows > 2:
         assert np.array_equal(got[1], want[1])
+
+
+def test_rmsnorm_softmax_rows_past_one_launch(rt):
+    """More rows than one launch's threads reach (2^25 at 64 threads a row): the second launch continues where
+    the first ended."""
+    rows, cols, part = 2 ** 25 + 5, 2, 4096
+    rng = np.random.default_rng(25)
+    x, g = bf16(rng, 3 * part * cols), bf16(rng, cols, 0.1, 1.0)
+    whole = np.resize(x, rows * cols)
+    out = rt.alloc(rows * cols * 2)
+    print(f"rmsnorm_softmax past one launch {rows}x{cols}", flush=True)
+    rt.rmsnorm_softmax(out, rt.upload(whole), rt.upload(g), rows, cols, 1e-6)
+    got = out.read(np.uint16).reshape(rows, cols)
+    want = rmsnorm_softmax_numpy(x, g, 3 * part, cols, 1e-6)
+    close_chain(emu.bf16_to_f32(got[:3 * part].ravel()).reshape(-1, cols), want, hard=rmsnorm_bound(x, g, 3 * part, cols, 1e-6),
+                frac_beyond=1e-4)
+    assert np.array_equal(got, np.resize(got[:3 * part], got.shape))

@@ -1,0 +1,40 @@
+"""The host rules that choose kernel forms, tiles and launch pieces (furiosa-opt_amd/csrc/launch_rules.hpp),
+built with g++ and asked through tests/host_rules/rules.cpp. No GPU."""
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("rules") / "rules"
+    res = subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", f"-I{ROOT / 'furiosa-opt_amd' / 'csrc'}",
+                          str(ROOT / "tests" / "host_rules" / "rules.cpp"), "-o", str(exe)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-4000:]
+
+    def run(questions):
+        out = subprocess.run([str(exe)], input="\n".join(questions) + "\n", capture_output=True, text=True, timeout=60)
+        assert out.returncode == 0
+        return [line.strip() for line in out.stdout.splitlines()]
+    return run
+
+
+# rows, threads a row: around the first piece's end, and the shapes that one launch could not take (512
+# columns from 2^26 rows, 2048 from 2^24, 4096 x 64 threads)
+@pytest.mark.parametrize("rows, threads", [(1, 64), (2 ** 25 - 1, 64), (2 ** 25, 64), (2 ** 25 + 1, 64), (2 ** 26, 64),
+                                           (2 ** 26 + 5, 64), (2 ** 31 + 3, 64), (2 ** 24 + 1, 256), (2 ** 23, 512),
+                                           (2 ** 22 + 7, 1024), (155648, 16), (2 ** 31 - 1, 16)])
+def test_row_pieces_cover_the_rows_and_fit_a_launch(ask, rows, threads):
+    pieces = [tuple(map(int, p.split("+"))) for p in ask([f"pieces {rows} {threads}"])[0].split()]
+    at = 0
+    for first, count in pieces:
+        assert first == at and count > 0
+        assert -(-count // 16) * 16 * threads < 2 ** 32  # whole blocks of up to 16 rows
+        assert first % 64 == 0  # no block straddles two pieces
+        at += count
+    assert at == rows
