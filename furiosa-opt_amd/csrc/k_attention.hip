@@ -40,6 +40,7 @@
 // code only on a block that hides some key from one of its queries.
 #include <hip/hip_runtime.h>
 
+#include "launch_rules.hpp"
 #include "runtime.hpp"
 
 namespace fo {
@@ -657,24 +658,11 @@ void launch_attention_prefill(hipStream_t s, uint16_t* out, const uint16_t* q, c
   require(ht * nqb < (1ll << 31) && (seq + 2 * kBN) * head_dim * 2 < (1ll << 31), "attention: shape too large");
   dim3 grid((unsigned)(ht * nqb));
   const float inv_sd = 1.0f / sqrt_d;
-  // Which form, by the workgroups each would have (WG64 and WG128: a workgroup per 64 or 128 queries of a
-  // head). Kernel alone in a recorded graph, D = 128 causal, us (one box):
-  //     heads, seq    WG64   2 x 4 groups    WG128   4 x 2 groups    256 queries
-  //     1, 600          10       14.1            5       16.3            22.4
-  //     16, 600        160       15.5           80       17.3            23.2
-  //     16, 1024       256       21.0          128       24.9            34.5
-  //     64, 300        320       16.8          192       13.1            16.3
-  //     64, 600        640       31.6          320       21.4            26.6
-  //     32, 2048      1024       87            512       60.4            66.3
-  //     128, 512      1024       43            512       27.4            25.0
-  //     64, 2048      2048      174           1024      120             106.5
-  //     16, 64          16        7.4           16        7.0             7.1
-  // and D = 64 alike (16, 600: 10.3, 11.4, 17.1). A given row maximum keeps the 256-query form.
-  const int64_t wg64 = ht * ((seq + 63) / 64), wg128 = ht * ((seq + 127) / 128);
-  if (!row_max && wg64 <= 256 && seq > 64) {
+  const AttnForm form = row_max ? AttnForm::kQueries256 : attention_form(ht, seq, causal != 0);
+  if (form == AttnForm::kKeys4) {
     head_dim == 128 ? launch_split<128, 2, 4>(s, out, q, k, v, ht, seq, inv_sd, causal)
                     : launch_split<64, 2, 4>(s, out, q, k, v, ht, seq, inv_sd, causal);
-  } else if (!row_max && (wg128 <= 320 || (wg128 <= 512 && seq >= 1024))) {
+  } else if (form == AttnForm::kKeys2) {
     head_dim == 128 ? launch_split<128, 4, 2>(s, out, q, k, v, ht, seq, inv_sd, causal)
                     : launch_split<64, 4, 2>(s, out, q, k, v, ht, seq, inv_sd, causal);
   } else if (head_dim == 128)

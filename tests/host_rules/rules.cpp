@@ -17,6 +17,12 @@ int main() {
       in >> rows >> threads;
       fo::for_row_pieces(rows, threads, [](int64_t first, int64_t count) { std::printf("%lld+%lld ", (long long)first, (long long)count); });
       std::printf("\n");
+    } else if (rule == "attention") {
+      int64_t heads, seq;
+      int causal;
+      in >> heads >> seq >> causal;
+      const char* names[] = {"2x4", "4x2", "256"};
+      std::printf("%s\n", names[(int)fo::attention_form(heads, seq, causal != 0)]);
     } else {
       return 1;
     }

@@ -38,3 +38,16 @@ def test_row_pieces_cover_the_rows_and_fit_a_launch(ask, rows, threads):
         assert first % 64 == 0  # no block straddles two pieces
         at += count
     assert at == rows
+
+
+# heads, keys, causal -> form: both sides of each line, with the shapes whose second round of workgroups was
+# slower than the 256-query form (100 x 300, 20 x 2000 and 32 x 1200 without a mask)
+@pytest.mark.parametrize("heads, seq, causal, form", [
+    (1, 65, 1, "2x4"), (16, 1024, 1, "2x4"), (16, 1024, 0, "2x4"), (256, 64, 1, "4x2"), (16, 1025, 1, "4x2"),
+    (32, 1024, 0, "4x2"), (33, 1024, 0, "256"), (33, 1000, 1, "4x2"), (64, 600, 0, "256"), (64, 600, 1, "4x2"),
+    (65, 600, 1, "256"), (100, 300, 0, "256"), (100, 300, 1, "256"), (100, 385, 1, "256"), (80, 385, 1, "4x2"),
+    (86, 384, 1, "256"), (32, 1200, 0, "256"), (32, 1200, 1, "4x2"), (32, 2048, 1, "4x2"), (32, 2048, 0, "256"),
+    (33, 2048, 1, "256"), (20, 2000, 0, "256"), (320, 128, 0, "4x2"), (321, 128, 0, "256"), (300, 129, 1, "256"),
+    (128, 2048, 1, "256")])
+def test_attention_form(ask, heads, seq, causal, form):
+    assert ask([f"attention {heads} {seq} {causal}"]) == [form]
