@@ -9,9 +9,10 @@ from test_gpu_fused import attention_numpy, bf16, close_chain
 pytestmark = pytest.mark.gpu
 
 # (heads, seq): the 4 x 2 form up to 64 keys, the 2 x 4 form over several steps of 256 keys, then the 4 x 2 form (more
-# than 256 workgroups of 64 queries, at most 320 of 128), then just past it.
+# than 256 workgroups of 64 queries, at most 256 to 512 of 128 by length and mask), then the 256-query form: one
+# query block, several with a ragged last one.
 CASES = [(1, 1), (3, 31), (2, 32), (5, 33), (2, 63), (2, 64), (3, 65), (2, 129), (1, 255), (2, 256), (1, 257), (2, 511),
-         (1, 513), (1, 800), (257, 40), (100, 150), (64, 257), (52, 513), (36, 1025), (330, 90)]
+         (1, 513), (1, 800), (257, 40), (100, 150), (64, 257), (52, 513), (36, 1025), (330, 90), (170, 333), (110, 600)]
 
 
 @pytest.mark.parametrize("causal", [True, False])
@@ -35,10 +36,11 @@ def test_attention_split(rt, case, d, causal):
         close_chain(got[i], ref, frac_beyond=2e-3, hard=bound)
 
 
-def test_attention_split_growing_logits(rt):
+@pytest.mark.parametrize("h", [2, 110])  # the 2 x 4 form, and several blocks of the 256-query form
+def test_attention_split_growing_logits(rt, h):
     """Keys whose logits grow along the sequence, so every later block raises the running max by far
     more than the rescale margin, and queries that see only the first, small ones."""
-    h, s, d = 2, 600, 128
+    s, d = 600, 128
     rng = np.random.default_rng(9)
     q = np.abs(rng.standard_normal((h, s, d))).astype(np.float32)
     k = (rng.standard_normal((h, s, d)) * 0.1 + np.linspace(0.0, 3.0, s)[None, :, None]).astype(np.float32)
@@ -48,7 +50,7 @@ def test_attention_split_growing_logits(rt):
     rt.attention_prefill(out, rt.upload(q), rt.upload(k), rt.upload(v), 1, h, s, d, 11.313708, True)
     got = emu.bf16_to_f32(out.read(np.uint16)).reshape(h, s, d)
     # a causal row's own max: the chain over its visible keys alone (p rounds at that scale here)
-    for i in range(h):
+    for i in (0, h - 1):
         sl = slice(i * s * d, (i + 1) * s * d)
         for row in (0, 40, 64, 255, 256, 400, 599):
             n = row + 1
