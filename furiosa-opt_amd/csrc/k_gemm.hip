@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "launch_rules.hpp"
 #include "runtime.hpp"
 
 namespace fo {
@@ -1101,20 +1102,9 @@ void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, c
   FO_HIP(hipGetLastError());
 }
 
-// Tile choice, by how many tiles of each size the output has (T64, T128, T256; batches included)
-// on the 256 CUs. Measured on one box as the kernel alone in a recorded graph, bf16 -> bf16, us:
-//     M, N, K            64x64   128x128 4 stages   128x128 2 stages   256x256 (k_gemm4)
-//     500, 3072, 1024     10.0        12.9               15.3               38
-//     512, 4096, 4096     30.7        32.3               42.6               75      T64 = 512
-//     1024, 4096, 4096    58          42.5               48.1               76      T128 = 256
-//     2048, 4096, 4096   107          78.6               69.8               79      T128 = 512
-//     3000, 3000, 2992   140          92.6               95.6               81      T256 = 144
-//     2048, 8192, 1024    68          54                 44.8               37.5    T256 = 256
-// and the same order for i8. Hence: 64x64 (32 KiB of LDS a stage pair, two blocks a CU) up to two
-// tiles a CU; 128x128 with four stages in flight while one block a CU covers them; with two stages,
-// two blocks a CU, up to 512; past that 256x256: four waves of 128x128 in 16x16 MFMA tiles (k_gemm4)
-// for bf16 and i8, eight waves of 128x64 in 32x32 tiles (k_gemm) for the 8-bit floats, whose 32-byte
-// fragments have no 16x16 form here.
+// Tile choice (gemm_tile in launch_rules.hpp, with its figures): 256x256 is four waves of 128x128 in 16x16
+// MFMA tiles (k_gemm4) for bf16 and i8, eight waves of 128x64 in 32x32 tiles (k_gemm) for the 8-bit floats,
+// whose 32-byte fragments have no 16x16 form here.
 //
 // Up to 32 rows: 32x64 tiles of two waves, half the LDS traffic a stage (i8 16, 8192, 8192 15.8 us against
 // 18.0 for 64x64, bf16 16, 4096, 4096 11.9 against 13.6, each with its best number of blocks a tile).
@@ -1124,7 +1114,7 @@ void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, c
 // 14.0 with 2 against 11.6 with one.
 // FO_GEMM_TILE overrides the tile for measurement: 32 (32x64), 64, 128, 1284 (128x128, four stages), 2568 (k_gemm,
 // 256x256) or 4128 (k_gemm4).
-int64_t tiles_of(const GemmDesc& d, int64_t t) { return ((d.M + t - 1) / t) * ((d.N + t - 1) / t) * d.batch; }
+int64_t tiles_of(const GemmDesc& d, int64_t t) { return fo::tiles_of(d.M, d.N, d.batch, t, t); }
 
 // Blocks sharing a tile of `rows` x 64, for the least estimated time: a stage of k takes 0.23 us when a
 // block has its CU to itself, sharing costs 2.2 us and, for the partial accumulators, 17 ns (64 rows) or
@@ -1167,8 +1157,9 @@ void gemm_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, void
   }();
   constexpr bool k16 = (KIND == kBf16 || KIND == kI8) && OUT <= 4;  // kinds with a 16x16 MFMA form here
   const int64_t t64 = tiles_of(d, 64);
-  int choice = forced;
-  if (!choice) choice = d.M <= 32 && t64 <= 512 ? 32 : t64 <= 512 ? 64 : tiles_of(d, 128) <= 256 ? 1284 : tiles_of(d, 256) < 144 ? 128 : k16 ? 4128 : 2568;
+  constexpr bool f8 = KIND == kF8E4M3 || KIND == kF8E5M2;
+  int choice = forced ? forced : gemm_tile(d.M, d.N, d.K, d.batch, f8);
+  if (choice == kTile256) choice = k16 ? 4128 : 2568;
   if constexpr (k16) {
     // four waves of 128x128 (16x16 MFMA tiles), 128-byte stages, A and B double-buffered. (A
     // triple-buffered, running a stage further ahead than B in the 32 KiB of LDS left over, measured

@@ -23,6 +23,11 @@ int main() {
       in >> heads >> seq >> causal;
       const char* names[] = {"2x4", "4x2", "256"};
       std::printf("%s\n", names[(int)fo::attention_form(heads, seq, causal != 0)]);
+    } else if (rule == "gemm") {
+      std::string type;
+      int64_t batch, m, n, k;
+      in >> type >> batch >> m >> n >> k;
+      std::printf("%d\n", (int)fo::gemm_tile(m, n, k, batch, type == "f8"));
     } else {
       return 1;
     }
