@@ -1169,7 +1169,7 @@ void gemm_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, void
   constexpr bool k16 = (KIND == kBf16 || KIND == kI8) && OUT <= 4;  // kinds with a 16x16 MFMA form here
   const int64_t t64 = tiles_of(d, 64);
   constexpr bool f8 = KIND == kF8E4M3 || KIND == kF8E5M2;
-  int choice = forced ? forced : gemm_tile(d.M, d.N, d.K, d.batch, f8);
+  int choice = forced ? forced : gemm_tile(d.M, d.N, d.K, d.batch, MfmaT<KIND>::EB, f8);
   if (choice == kTile256) choice = k16 ? 4128 : 2568;
   if constexpr (k16) {
     // four waves of 128x128 (16x16 MFMA tiles), 128-byte stages, A and B double-buffered. (A

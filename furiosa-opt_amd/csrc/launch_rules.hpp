@@ -47,6 +47,11 @@ inline AttnForm attention_form(int64_t heads, int64_t seq, bool causal) {
 //     bf16  500, 3072, 1024         10.0        12.9               15.3             38
 //     bf16  512, 4096, 4096         30.7        32.3               42.6             75      T64 = 512
 //     bf16  1024, 4096, 4096        58          39.3               48.6             76      T128 = 256
+//     bf16  1024, 4096, 512         13.1        10.4               10.0             20      8 stages of 128 bytes of k
+//     bf16  343, 5584, 384           9.7         8.6                8.2             26      6
+//     i8    900, 3500, 1024         13.7        11.5               11.2             24      8
+//     i8    1024, 4096, 1536         -          14.1               14.4              -      12
+//     bf16  1024, 4096, 1536         -          18.5               22.4              -      24
 //     bf16  2048, 4096, 4096       104          75.0               66.9             80      T128 = 512, T256 = 128
 //     f8    2048, 4096, 4096        58          45.7               36.6             52
 //     bf16  1500, 5500, 1024        37.9        39.9               35.2             44      T128 = 516, T256 = 132
@@ -57,17 +62,17 @@ inline AttnForm attention_form(int64_t heads, int64_t seq, bool causal) {
 //     f8    1500, 5500, 2048        34.9        39.4               35.0             32.0
 //     bf16  2048, 8192, 1024        68          54                 44.8             37.5    T256 = 256
 // Hence: 64x64 (32 KiB of LDS a stage pair, two blocks a CU) up to two tiles a CU; 128x128 with four stages
-// in flight while one block a CU covers them; with two stages, two blocks a CU, up to 512; past that
-// 256x256, but for the first, mostly empty round of them over a short K (1024 elements; 512 of the 8-bit
+// in flight while one block a CU covers them and K has stages enough to pay for filling four; with two
+// stages, two blocks a CU, up to 512; past that 256x256, but for the first, mostly empty round of them over a short K (1024 elements; 512 of the 8-bit
 // floats, whose 256x256 form is the faster one).
 enum GemmTile { kTile32x64 = 32, kTile64 = 64, kTile128 = 128, kTile128Deep = 1284, kTile256 = 256 };
 inline int64_t tiles_of(int64_t m, int64_t n, int64_t batch, int64_t tm, int64_t tn) {
   return ((m + tm - 1) / tm) * ((n + tn - 1) / tn) * batch;
 }
-inline GemmTile gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool f8) {
+inline GemmTile gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes, bool f8) {
   const int64_t t64 = tiles_of(m, n, batch, 64, 64), t128 = tiles_of(m, n, batch, 128, 128);
   if (t64 <= 512) return m <= 32 ? kTile32x64 : kTile64;
-  if (t128 <= 256) return kTile128Deep;
+  if (t128 <= 256 && (k * elem_bytes + 127) / 128 >= 12) return kTile128Deep;
   if (t128 <= 512) return kTile128;
   if (tiles_of(m, n, batch, 256, 256) < 144 && k <= (f8 ? 512 : 1024)) return kTile128;
   return kTile256;

@@ -27,7 +27,7 @@ int main() {
       std::string type;
       int64_t batch, m, n, k;
       in >> type >> batch >> m >> n >> k;
-      std::printf("%d\n", (int)fo::gemm_tile(m, n, k, batch, type == "f8"));
+      std::printf("%d\n", (int)fo::gemm_tile(m, n, k, batch, type == "bf16" ? 2 : 1, type == "f8"));
     } else {
       return 1;
     }
