@@ -1117,7 +1117,7 @@ void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, c
 // MFMA tiles (k_gemm4) for bf16 and i8, eight waves of 128x64 in 32x32 tiles (k_gemm) for the 8-bit floats,
 // whose 32-byte fragments have no 16x16 form here.
 //
-// Up to 32 rows: 32x64 tiles of two waves, half the LDS traffic a stage (i8 16, 8192, 8192 15.8 us against
+// Up to 32 rows, at any number of tiles: 32x64 tiles of two waves, half the LDS traffic a stage (i8 16, 8192, 8192 15.8 us against
 // 18.0 for 64x64, bf16 16, 4096, 4096 11.9 against 13.6, each with its best number of blocks a tile).
 //
 // Few tiles leave CUs idle while each walks all of K, so blocks share a tile (splits_of): 64, 1024, 4096

@@ -64,16 +64,29 @@ inline AttnForm attention_form(int64_t heads, int64_t seq, bool causal) {
 // Hence: 64x64 (32 KiB of LDS a stage pair, two blocks a CU) up to two tiles a CU; 128x128 with four stages
 // in flight while one block a CU covers them and K has stages enough to pay for filling four; with two
 // stages, two blocks a CU, up to 512; past that 256x256, but for the first, mostly empty round of them over a short K (1024 elements; 512 of the 8-bit
-// floats, whose 256x256 form is the faster one).
+// floats, whose 256x256 form is the faster one). An output side of up to 32, 64 or 128 keeps the tile as small
+// at any number of tiles, the rest of a larger one being padding (batch x M, N, K):
+//     types                       32x64   64x64   128x128 2 stages   256x256
+//     bf16  16, 155648, 1024       60.1    65.2         70.2           87.3
+//     bf16  32, 65536, 256          9.2     9.4          9.3           16.2
+//     bf16  64, 40000, 1024          -     18.1         19.4           34.2
+//     bf16  128, 65536, 1024         -     37.4         26.5           36.2
+//     i8    100, 40000, 1024         -     20.0         16.1           24.9
+//     bf16  520 x 16, 64, 256        5.8    7.7         11.2           34.2
+//     f8    600 x 64, 64, 512        -     10.9         16.0           27.3
+//     bf16  300 x 100, 100, 256      -     16.3         10.7           45.3
 enum GemmTile { kTile32x64 = 32, kTile64 = 64, kTile128 = 128, kTile128Deep = 1284, kTile256 = 256 };
 inline int64_t tiles_of(int64_t m, int64_t n, int64_t batch, int64_t tm, int64_t tn) {
   return ((m + tm - 1) / tm) * ((n + tn - 1) / tn) * batch;
 }
 inline GemmTile gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes, bool f8) {
-  const int64_t t64 = tiles_of(m, n, batch, 64, 64), t128 = tiles_of(m, n, batch, 128, 128);
-  if (t64 <= 512) return m <= 32 ? kTile32x64 : kTile64;
+  const int64_t t64 = tiles_of(m, n, batch, 64, 64), t128 = tiles_of(m, n, batch, 128, 128), side = std::min(m, n);
+  // Batches are the launch's second dimension; the first one's threads have to fit 32 bits.
+  auto fits = [&](int64_t tm, int64_t tn, int64_t threads) { return tiles_of(m, n, 1, tm, tn) * threads < (1ll << 32); };
+  if (m <= 32 && fits(32, 64, 128)) return kTile32x64;
+  if ((t64 <= 512 || side <= 64) && fits(64, 64, 256)) return kTile64;
   if (t128 <= 256 && (k * elem_bytes + 127) / 128 >= 12) return kTile128Deep;
-  if (t128 <= 512) return kTile128;
+  if ((t128 <= 512 || side <= 128) && fits(128, 128, 256)) return kTile128;
   if (tiles_of(m, n, batch, 256, 256) < 144 && k <= (f8 ? 512 : 1024)) return kTile128;
   return kTile256;
 }

@@ -36,9 +36,11 @@ def product(a, b):
 
 
 # One tile and its remainders, K below, at and past a stage; then sizes where 8, 4, 3 and 2 blocks
-# share a tile (uneven runs of stages, a partial last one); then the first and last sizes of each tile.
+# share a tile (uneven runs of stages, a partial last one); then the first and last sizes of each tile, four
+# stages in flight among them, and small sides past 512 tiles.
 SIZES = [(8, 8, 16), (64, 64, 64), (65, 63, 80), (9, 70, 6160), (64, 64, 12304), (130, 200, 4624), (128, 1030, 2080),
-         (257, 8136, 512), (520, 4096, 144), (2048, 2049, 96), (2300, 4090, 64), (3072, 3000, 48)]
+         (257, 8136, 512), (520, 4096, 144), (2048, 2049, 96), (2300, 4090, 64), (3072, 3000, 48),
+         (257, 8136, 1552), (20, 33000, 80), (33010, 63, 48), (33000, 40, 272), (70, 70000, 48)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
@@ -98,3 +100,20 @@ def test_w8a8_shared_tiles(rt, size):
         rt.gemm_w8a8_dequant(other, None, a, w, s, m, n, k)
         assert np.array_equal(other.read(np.uint16), want)
     graph.free()
+
+
+# Batches of products smaller than a tile, more of them than 512 tiles.
+@pytest.mark.parametrize("size", [(520, 16, 64, 80), (600, 63, 40, 48), (530, 100, 72, 160)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("types", list(TYPES))
+def test_gemm_tiles_batches_exact(rt, size, types):
+    b, m, n, k = size
+    in_t, out_t = TYPES[types]
+    rng = np.random.default_rng(sum(size))
+    av, a = operands(rng, in_t, b * m, k)
+    bv, w = operands(rng, in_t, b * n, k)
+    want = narrowed(np.matmul(av.reshape(b, m, k).astype(np.float64), bv.reshape(b, n, k).astype(np.float64).transpose(0, 2, 1)), out_t)
+    maps = [fh.m(t, B=b, M=m, N=n, K=k) for t in ("B, M, K", "B, N, K", "B, M, N, K", "B, M, N")]
+    out = rt.upload(np.full(b * m * n, 0x5A, dtype=fh.NP_DTYPE[out_t]))
+    print(f"gemm tiles batches {size} {types}", flush=True)
+    rt.contraction(out, rt.upload(a), rt.upload(w), in_t, out_t, *maps)
+    assert np.array_equal(out.read(out_t).ravel(), want.ravel())

@@ -61,6 +61,11 @@ def test_attention_form(ask, heads, seq, causal, form):
     ("i8 1 900 3500 1409", 1284), ("f8 1 343 5584 384", 128), ("bf16 1 1100 4096 4096", 128), ("bf16 1 2048 4096 4096", 128), ("f8 1 2048 4096 4096", 128),
     ("i8 1 2048 4096 8192", 128), ("bf16 1 1500 5500 1024", 128), ("bf16 1 1500 5500 1025", 256), ("bf16 1 2304 3840 2048", 256),
     ("i8 1 1500 5500 1024", 128), ("i8 1 1500 5500 4096", 256), ("f8 1 1500 5500 512", 128), ("f8 1 1500 5500 2048", 256),
-    ("bf16 16 600 600 128", 128), ("bf16 1 2200 3900 1024", 256), ("bf16 1 4096 4096 4096", 256), ("i8 1 2048 8192 8192", 256)])
+    ("bf16 16 600 600 128", 128), ("bf16 1 2200 3900 1024", 256), ("bf16 1 4096 4096 4096", 256), ("i8 1 2048 8192 8192", 256),
+    # a small side keeps its tile past 512 tiles, while a launch can hold them
+    ("bf16 1 16 155648 1024", 32), ("bf16 520 16 64 256", 32), ("bf16 1 64 40000 1024", 64), ("i8 1 40000 64 1024", 64),
+    ("f8 600 64 64 512", 64), ("bf16 1 65 40000 1024", 128), ("bf16 300 100 100 256", 128), ("i8 1 128 155648 8192", 128),
+    ("bf16 1 129 155648 1024", 256), ("bf16 1 8 2147483647 16", 256), ("bf16 1 40 2147483647 16", 256),
+    ("bf16 1 40 1073741760 16", 64), ("bf16 1 32 2147483520 16", 32), ("bf16 1 40 2147483520 16", 128), ("bf16 1 129 2147483647 16", 256)])
 def test_gemm_tile(ask, shape, tile):
     assert ask([f"gemm {shape}"]) == [str(tile)]
