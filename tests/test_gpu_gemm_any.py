@@ -70,3 +70,20 @@ def test_gemm_any_alignment_layouts(rt, layout, k, types):
     rt.contraction(out, rt.upload(store(l_t, av, s["M"])), rt.upload(store(r_t, bv, s["N"])), in_t, out_t,
                    *(fh.m(t, **s) for t in (l_t, r_t, pre, o_t)))
     assert np.array_equal(out.read(out_t).ravel(), narrowed(np.ascontiguousarray(acc).ravel(), out_t).ravel())
+
+
+# More products or columns than 512 tiles of 64x64, a side of at most 64: the smaller tile.
+@pytest.mark.parametrize("size", [(520, 32, 31, 65), (70, 64, 520, 71), (1, 16, 33001, 129)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("types", ["bf16-f32", "i8-i32"])
+def test_gemm_any_many_small_exact(rt, size, types):
+    b, m, n, k = size
+    in_t, out_t = TYPES[types]
+    rng = np.random.default_rng(sum(size))
+    av, a = operands(rng, in_t, b * m, k)
+    bv, w = operands(rng, in_t, b * n, k)
+    want = narrowed(np.matmul(av.reshape(b, m, k).astype(np.float64), bv.reshape(b, n, k).astype(np.float64).transpose(0, 2, 1)), out_t)
+    maps = [fh.m(t, B=b, M=m, N=n, K=k) for t in ("B, M, K", "B, N, K", "B, M, N, K", "B, M, N")]
+    out = rt.upload(np.full(b * m * n, 0x5A, dtype=fh.NP_DTYPE[out_t]))
+    print(f"gemm any many {size} {types}", flush=True)
+    rt.contraction(out, rt.upload(a), rt.upload(w), in_t, out_t, *maps)
+    assert np.array_equal(out.read(out_t).ravel(), want.ravel())

@@ -69,3 +69,11 @@ def test_attention_form(ask, heads, seq, causal, form):
     ("bf16 1 40 1073741760 16", 64), ("bf16 1 32 2147483520 16", 32), ("bf16 1 40 2147483520 16", 128), ("bf16 1 129 2147483647 16", 256)])
 def test_gemm_tile(ask, shape, tile):
     assert ask([f"gemm {shape}"]) == [str(tile)]
+
+
+# batch, m, n -> tile of the contraction off 16-byte rows; batches of small products went to 128x128 once
+@pytest.mark.parametrize("shape, tile", [("1 333 1000", 64), ("1 1500 2000", 128), ("2000 32 32", 64), ("600 64 200", 64), ("600 65 70", 128),
+                                         ("1 16 155648", 64), ("1 8 1073741760", 64), ("1 8 1073741888", 128),
+                                         ("1 8 2147483647", 0)])
+def test_gemm_any_tile(ask, shape, tile):
+    assert ask([f"gemm_any {shape}"]) == [str(tile)]
