@@ -12,6 +12,7 @@
 
 #include <algorithm>
 
+#include "launch_rules.hpp"
 #include "runtime.hpp"
 
 namespace fo {
@@ -496,19 +497,11 @@ void launch_mlp(hipStream_t s, int32_t* pred, uint16_t* logits, const uint16_t* 
                      ((uintptr_t)w1 % 16) == 0 && lds_split <= 160 * 1024;
   const size_t lds = (size_t)(in_f + hidden + out_f) * sizeof(float);
   require(split || lds <= 64 * 1024, "mlp: layer widths exceed the LDS budget");
-  // A row per block while every row can have a CU: producers and folders (k_mlp_split) where the shape
-  // fits them, two blocks a CU up to 64 units wide (446 x 392 x 19 x 38 13.5 us against 14.5 on k_mlp_rows,
-  // 512 x 784 x 32 x 10 18.9 against 20.8, x 64 x 10 21.3 against 22.2; x 128 x 10 26.3 against 24.2). Past
-  // that, the fewest rows a block (a power of two) that leave one block a CU. Kernel
-  // alone in a recorded graph, batch x inputs x hidden x outputs, us, before -> k_mlp_rows:
-  //     256 x 784 x 128 x 10      14.6 (split) -> 23      4096 x 784 x 128 x 10     184 (split) -> 45
-  //     512 x 784 x 128 x 10      26.5 (split) -> 24      1104 x 270 x 147 x 33    32.6 (k_mlp) -> 24
-  //     1024 x 784 x 128 x 10     49.5 (split) -> 28      4096 x 1024 x 512 x 64    955 (k_mlp) -> 185
-  //     59 x 271 x 401 x 64       40.3 (k_mlp) -> 28      2 x 73 x 23 x 34          7.3 (k_mlp) -> 8.8
-  // so small layers the producers do not take keep a thread per fold (k_mlp).
-  const bool small = batch <= 256 && hidden <= 256 && in_f + hidden <= 128;
-  const bool row_per_block = split && batch <= (hidden <= 64 ? 512 : 256);
-  if (!row_per_block && !small) {
+  // Rows of k_mlp_rows: the fewest a block (a power of two) that leave one block a CU. Kernel alone in a recorded
+  // graph, batch x inputs x hidden x outputs, us, a row a block -> k_mlp_rows:
+  //     1024 x 784 x 128 x 10     46.7 (split) -> 26      1104 x 270 x 147 x 33    32.6 (k_mlp) -> 24
+  //     4096 x 784 x 128 x 10    179.7 (split) -> 42      4096 x 1024 x 512 x 64    955 (k_mlp) -> 185
+  if (mlp_form(batch, in_f, hidden, split) == MlpForm::kRows) {
     MlpArgs g{pred, logits, x, w1, b1, w2, b2, (int32_t)batch, (int32_t)in_f, (int32_t)hidden, (int32_t)out_f, 0, 0, 0, 0};
     if (batch > 2048 && mlp_rows_launch<16>(s, g)) return;
     if (batch > 1024 && mlp_rows_launch<8>(s, g)) return;

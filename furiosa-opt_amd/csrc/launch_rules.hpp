@@ -100,4 +100,47 @@ inline int gemm_any_tile(int64_t m, int64_t n, int64_t batch) {
   return fits(128) ? 128 : 0;
 }
 
+// The MLP's forms: a row a block with a thread per fold (k_mlp) or, where the shape fits them, producer and
+// folder waves (k_mlp_split, `split`); or several rows a block (k_mlp_rows). Kernel alone in a recorded graph, one
+// box, us, one row a block / k_mlp_rows:
+//     k_mlp_split, batch:         257           320-400         512          513
+//     64, 65, 10                6.7 / 7.6      7.2 / 7.7      7.3 / 7.8        -
+//     400, 72, 10              13.8 / 15.4    14.3 / 15.5    14.4 / 15.5       -
+//     64, 88, 10                8.7 / 7.9      9.2 / 8.0      9.3 / 8.0        -
+//     784, 100, 10             22.3 / 22.9    23.0 / 23.0    23.1 / 23.0       -
+//     256, 112, 10             12.1 / 12.3    12.6 / 12.4    12.7 / 12.5       -
+//     64, 128, 10               7.6 / 8.1      8.0 / 8.1      8.2 / 8.2        -
+//     784, 128, 10             23.5 / 22.5    24.2 / 22.5    24.4 / 22.6   34.4 / 26.0
+//     1024, 136, 10            31.2 / 33.4    32.1 / 33.2    32.3 / 33.3       -
+//     784, 160, 10             27.9 / 28.3    28.8 / 28.6    29.1 / 28.6   41.2 / 30.2
+//     64, 16, 10                6.7 / -        7.2 / -        7.3 / -       9.4 / 6.7
+// so a second block a CU still pays, but for 105 to 128 units (the widest two folder waves hold) of a long row, or
+// with more than 16 units past whole runs of 32 (the second layer adds those one LDS read at a time).
+//     k_mlp, batch:               1             64-256         320-512       600-1024     1500      2048
+//     75, 25, 10                5.7 / -        6.4 / -        6.7 / 7.8     6.4 / 8.1   8.1 / 8.4   7.7 / 8.4
+//     105, 16, 10               6.1 / -        7.0 / -        9.0 / 8.4     7.1 / 8.7   8.5 / 9.1   8.2 / 9.2
+//     34, 102, 10               6.9 / 8.1      7.7 / 8.6      9.7 / 8.9     8.1 / 9.0  10.4 / 9.4  10.8 / 9.5
+//     75, 75, 50                8.4 / 9.5      9.0 / 10.0    10.0 / 10.5   10.0 / 11.4 12.9 / 11.3 13.8 / 11.4
+//     134, 16, 10               7.3 / 8.2      8.3 / 8.7     10.8 / 9.0     8.4 / 9.1  10.0 / 9.5   9.6 / 9.5
+//     100, 100, 50              9.6 / 10.4    10.1 / 10.9    11.4 / 11.4   11.7 / 12.5 15.4 / 12.6 16.6 / 12.8
+//     50, 150, 10               8.7 / 9.8      9.7 / 10.4    12.5 / 10.6   11.0 / 10.8 14.4 / 12.3 16.6 / 12.4
+//     164, 16, 10               8.1 / 8.7      9.2 / 9.1     12.1 / 9.5     9.4 / 9.7  11.0 / 10.2 10.7 / 10.3
+//     70, 200, 5               10.5 / 11.5    11.9 / 11.9       -             -           -           -
+//     195, 65, 10              11.9 / 10.1    12.6 / 10.6    14.1 / 11.4   14.0 / 12.2 19.6 / 12.6 21.0 / 12.7
+// k_mlp's time is its two serial folds, an input costing about two hidden values; k_mlp_rows pays about 0.55 us
+// a chunk of 32 of either.
+enum class MlpForm { kThread, kSplit, kRows };
+inline MlpForm mlp_form(int64_t batch, int64_t in_f, int64_t hidden, bool split) {
+  if (split) {
+    const bool wide = (hidden > 104 && hidden <= 128 && in_f >= 256) || hidden % 32 > 16;
+    return batch <= (wide && hidden > 64 && hidden <= 128 ? 256 : 512) ? MlpForm::kSplit : MlpForm::kRows;
+  }
+  const int64_t folds = 2 * in_f + hidden;
+  const bool thread = batch <= 256    ? folds <= 344 && hidden <= 256
+                      : batch <= 512  ? folds <= 240 && hidden <= 80
+                      : batch <= 1024 ? folds <= 315 && hidden <= 128
+                                      : batch <= 2048 && folds <= 260 && hidden <= 64;
+  return thread ? MlpForm::kThread : MlpForm::kRows;
+}
+
 }  // namespace fo

@@ -32,6 +32,12 @@ int main() {
       int64_t batch, m, n;
       in >> batch >> m >> n;
       std::printf("%d\n", fo::gemm_any_tile(m, n, batch));
+    } else if (rule == "mlp") {
+      int64_t batch, in_f, hidden;
+      int split;
+      in >> batch >> in_f >> hidden >> split;
+      const char* names[] = {"thread", "split", "rows"};
+      std::printf("%s\n", names[(int)fo::mlp_form(batch, in_f, hidden, split != 0)]);
     } else {
       return 1;
     }
