@@ -9,11 +9,10 @@
 // reference's bf16 rule (float/bf16.rs:16-40: a subnormal reads as a signed zero); the products
 // and sums themselves are IEEE f32, subnormal results included. The parallelism is across cells,
 // and the chain of K dependent adds per cell bounds a small GEMV, HBM a large one. Two kernels:
-//   * k_gemv_fold (K <= 4096): a block of four waves owns 16 or 32 cells. Waves 1-3 stream the weight
+//   * k_gemv_fold (K <= 4096): a block owns 16 or 32 cells with three producer waves, or 64 with six. They stream the weight
 //     rows from HBM (16-byte loads, four stages in flight) and write the exact f32 products of each
 //     96-element stage to LDS; wave 0 folds the previous stage's products, one cell per lane, so its
-//     instruction stream is one LDS read per four adds. (A 64-cell block needed six producer waves to
-//     keep up with the folder, and their LDS traffic slowed it.) The producer waves run with subnormal inputs
+//     instruction stream is one LDS read per four adds. The producer waves run with subnormal inputs
 //     flushed and subnormal results kept (the MODE register is per wave): the reference's widen of
 //     a subnormal weight to zero, then an IEEE product. The folding wave keeps full IEEE behaviour.
 //   * k_gemv_bf16 (any K): R cells per block, the rows staged through LDS by all waves and folded by
@@ -127,7 +126,6 @@ __global__ void __launch_bounds__(kGemvThreads) k_gemv_bf16(Out* __restrict__ ou
 
 constexpr int kFoldKC = 96;                         // k elements per stage
 constexpr int kFoldCPR = kFoldKC / 8;               // 16-byte chunks per row per stage
-constexpr int kFoldProducers = 192;                 // threads of waves 1-3
 constexpr int kFoldPS = kFoldKC + 4;  // product row stride in floats: 16 lanes' b128 reads cover 64 banks once
 constexpr int kFoldMaxK = 4096;       // x is staged whole in LDS
 constexpr int kFoldDepth = 4;         // stages of weight loads in flight per producer
@@ -139,13 +137,13 @@ constexpr int kDenormFlushIn = 2;
 
 // XF32: x is f32 data standing for the widen of its deferred bf16 narrow (the runtime's deferred
 // casts); each element is rounded to bf16 by the narrow's rule and widened as it is staged.
-// R: cells per block, one per lane of wave 0.
-template <int R, typename Out, bool XF32>
-__global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restrict__ out, const void* __restrict__ x,
+// R: cells per block, one per lane of wave 0. PROD: producer threads, waves 1 to PROD / 64.
+template <int R, int PROD, typename Out, bool XF32>
+__global__ void __launch_bounds__(64 + PROD) k_gemv_fold(Out* __restrict__ out, const void* __restrict__ x,
                                                    const uint16_t* __restrict__ w, int64_t N, int K, int64_t ldw,
                                                    int64_t ldo) {
-  constexpr int kPer = R * kFoldCPR / kFoldProducers;  // chunks per producer per stage
-  static_assert(R * kFoldCPR % kFoldProducers == 0, "producer chunks must divide evenly");
+  constexpr int kPer = R * kFoldCPR / PROD;  // chunks per producer per stage
+  static_assert(R * kFoldCPR % PROD == 0, "producer chunks must divide evenly");
   __shared__ __attribute__((aligned(16))) float P[2][R * kFoldPS];
   __shared__ __attribute__((aligned(16))) float xs[kFoldMaxK];
   const int t = threadIdx.x;
@@ -163,13 +161,13 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
   // The producers are a whole number of rows, so all of a producer's chunks share a column, and one read
   // of x's eight values serves them (with 64 cells a block, a read per chunk kept the LDS pipe as busy
   // as the fold: K = 1024 7.0 -> 6.3 us, 3072 15.7 -> 14.2, the 155,648-row head 62 -> 60).
-  static_assert(kFoldProducers % kFoldCPR == 0, "a producer's chunks share a column");
+  static_assert(PROD % kFoldCPR == 0, "a producer's chunks share a column");
   const uint16_t* wrow[kPer];
   int poff[kPer];
   const int pcol = (p % kFoldCPR) * 8;
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
-    const int row = (p + u * kFoldProducers) / kFoldCPR;
+    const int row = (p + u * PROD) / kFoldCPR;
     poff[u] = row * kFoldPS + pcol;
     wrow[u] = w + min(n0 + row, N - 1) * ldw;
   }
@@ -183,11 +181,11 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
   };
   if (!folder) {
     __builtin_amdgcn_s_setreg(kModeDenormF32, kDenormFlushIn);
-    constexpr int kXPer = (kFoldMaxK / 8 + kFoldProducers - 1) / kFoldProducers;  // x chunks per producer (3)
+    constexpr int kXPer = (kFoldMaxK / 8 + PROD - 1) / PROD;  // x chunks per producer (3)
     uint4 xv[kXPer][XF32 ? 2 : 1];
 #pragma unroll
     for (int u = 0; u < kXPer; ++u) {
-      const int c = min(p + u * kFoldProducers, xchunks - 1);
+      const int c = min(p + u * PROD, xchunks - 1);
       if constexpr (XF32) {
         xv[u][0] = *((const uint4*)((const float*)x + 8 * c));
         xv[u][1] = *((const uint4*)((const float*)x + 8 * c) + 1);
@@ -199,7 +197,7 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
     for (int j = 0; j < kFoldDepth; ++j) load(j, reg[j]);
 #pragma unroll
     for (int u = 0; u < kXPer; ++u) {  // the reference widen of x
-      const int c = p + u * kFoldProducers;
+      const int c = p + u * PROD;
       if (c < xchunks) {
         uint16_t h[8];
         if constexpr (XF32) {
@@ -292,17 +290,17 @@ __global__ void __launch_bounds__(64 + kFoldProducers) k_gemv_fold(Out* __restri
   if (t < R && n0 + t < N) out[(n0 + t) * ldo] = narrow_out<Out>(acc);
 }
 
-template <int R, typename Out>
+template <int R, int PROD, typename Out>
 void gemv_fold(hipStream_t s, Out* out, const void* x, bool x_f32, const uint16_t* w, int64_t N, int64_t K,
                int64_t ldw, int64_t ldo) {
-  static_assert((64 + kFoldProducers) % R == 0, "threads a row");
-  for_row_pieces(N, (64 + kFoldProducers) / R, [&](int64_t n, int64_t rows) {
-    const dim3 grid((unsigned)((rows + R - 1) / R)), block(64 + kFoldProducers);
+  static_assert(64 + PROD <= 16 * R, "threads a row");
+  for_row_pieces(N, 16, [&](int64_t n, int64_t rows) {
+    const dim3 grid((unsigned)((rows + R - 1) / R)), block(64 + PROD);
     if (x_f32)
-      hipLaunchKernelGGL((k_gemv_fold<R, Out, true>), grid, block, 0, s, out + n * ldo, x, w + n * ldw, rows, (int)K,
+      hipLaunchKernelGGL((k_gemv_fold<R, PROD, Out, true>), grid, block, 0, s, out + n * ldo, x, w + n * ldw, rows, (int)K,
                          ldw, ldo);
     else
-      hipLaunchKernelGGL((k_gemv_fold<R, Out, false>), grid, block, 0, s, out + n * ldo, x, w + n * ldw, rows, (int)K,
+      hipLaunchKernelGGL((k_gemv_fold<R, PROD, Out, false>), grid, block, 0, s, out + n * ldo, x, w + n * ldw, rows, (int)K,
                          ldw, ldo);
   });
   FO_HIP(hipGetLastError());
@@ -338,20 +336,14 @@ void launch_gemv(hipStream_t s, void* out, const void* x, const void* w, fo_dtyp
   require(!x_f32 || gemv_takes_f32_x(K), "gemv: an f32 x through its bf16 narrow takes K <= 4096");
   const uint16_t *xp = (const uint16_t*)x, *wp = (const uint16_t*)w;
   if (K <= kFoldMaxK) {
-    // 16 cells a block while the 256 CUs each take at most one block, else 32: fewer cells leave the LDS
-    // pipe to the fold (16 rows of reads and products a stage, not 64) and spread a small N over more CUs.
-    // Kernel alone in a recorded graph, N x K, us, 64 cells and six producer waves / 32 and three / 16 and
-    // three: 1024 x 1024 6.45 / 5.82 / 5.63; 3072 x 1024 6.58 / 5.90 / 5.73; 1024 x 3072 14.6 / 12.4 / 12.2;
-    // 155648 x 1024 60.9 / 59.1 / 70.6. (32 cells and six waves: 5.94, 6.08, 13.4, 70.6.)
-    const bool few = N <= 16 * 256;
-    if (out_t == FO_F32 && few)
-      gemv_fold<16>(s, (float*)out, x, x_f32, wp, N, K, ldw, ldo);
-    else if (out_t == FO_F32)
-      gemv_fold<32>(s, (float*)out, x, x_f32, wp, N, K, ldw, ldo);
-    else if (few)
-      gemv_fold<16>(s, (uint16_t*)out, x, x_f32, wp, N, K, ldw, ldo);
-    else
-      gemv_fold<32>(s, (uint16_t*)out, x, x_f32, wp, N, K, ldw, ldo);
+    auto run = [&](auto* o) {
+      switch (gemv_cells(N, K)) {
+        case 16: return gemv_fold<16, 192>(s, o, x, x_f32, wp, N, K, ldw, ldo);
+        case 32: return gemv_fold<32, 192>(s, o, x, x_f32, wp, N, K, ldw, ldo);
+        default: return gemv_fold<64, 384>(s, o, x, x_f32, wp, N, K, ldw, ldo);
+      }
+    };
+    out_t == FO_F32 ? run((float*)out) : run((uint16_t*)out);
     return;
   }
   // Rows per block: 64 where that still gives 512 blocks, else fewer so a small N spreads out.

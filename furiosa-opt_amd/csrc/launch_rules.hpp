@@ -143,4 +143,30 @@ inline MlpForm mlp_form(int64_t batch, int64_t in_f, int64_t hidden, bool split)
   return thread ? MlpForm::kThread : MlpForm::kRows;
 }
 
+// Cells a block of the folded GEMV (K up to 4096): 16 or 32 with three producer waves, or 64 with six. Fewer cells
+// leave the LDS pipe to the fold and spread a small N over more CUs; but a CU holds three blocks of 32 (by their
+// LDS: 24576 rows a round of the chip) or two of 64 (32768 rows), and a second block on a CU slows the first.
+// Kernel alone in a recorded graph, one box, us, 16 / 32 / 64:
+//     N             K = 64              512                 1024                2048                4096
+//     4097      3.0 / 3.2 / 3.3     4.3 / 4.5 / 4.8     5.9 / 5.9 / 6.6     9.8 / 9.7 / 10.6   17.2 / 16.0 / 18.7
+//     8192      3.2 / 3.2 / 3.3     4.7 / 4.6 / 4.9     6.4 / 6.3 / 7.0    11.0 / 10.1 / 11.2  18.9 / 17.2 / 19.0
+//     10000     3.3 / 3.4 / 3.3     5.4 / 5.1 / 4.9     7.4 / 7.1 / 7.0    12.7 / 12.1 / 11.9  21.0 / 21.3 / 19.3
+//     16384     3.5 / 3.4 / 3.4     5.9 / 5.3 / 5.3     8.8 / 7.7 / 7.3    15.7 / 13.5 / 12.8  25.3 / 29.2 / 21.7
+//     18000     4.5 / 3.7 / 3.8     7.7 / 6.2 / 6.7    12.4 / 9.7 / 10.0   21.0 / 16.8 / 18.5  35.9 / 36.2 / 33.7
+//     24576     4.8 / 3.8 / 3.9     8.9 / 6.3 / 6.9    14.6 / 10.2 / 10.3  23.8 / 19.3 / 19.6  40.3 / 36.8 / 34.6
+//     32768     5.2 / 5.1 / 4.0    10.5 / 9.2 / 7.1    16.9 / 14.1 / 13.3  27.9 / 24.3 / 21.8  47.8 / 48.3 / 41.1
+//     40000     6.4 / 5.6 / 5.4    13.7 / 12.2 / 10.9  20.0 / 16.5 / 17.0  34.2 / 27.7 / 29.3          -
+//     49152     7.1 / 5.9 / 5.5    15.5 / 13.2 / 11.8  23.0 / 18.7 / 17.7  39.9 / 32.9 / 30.4          -
+//     65536     8.8 / 7.7 / 6.3    19.4 / 16.4 / 15.1  29.3 / 23.5 / 22.6  51.3 / 43.0 / 40.1          -
+//     98304    12.2 / 10.0 / 9.7   26.9 / 21.6 / 21.6  41.0 / 31.6 / 33.7          -                   -
+//     155648   18.2 / 15.3 / 13.7  39.4 / 31.2 / 30.3  66.2 / 54.3 / 55.9          -                   -
+inline int gemv_cells(int64_t n, int64_t k) {
+  if (n <= 4096) return 16;
+  if (n <= 8192) return 32;
+  if (n <= 16384) return 64;
+  if (n <= 24576) return k <= 3584 ? 32 : 64;
+  if (n <= 32768 || k < 768) return 64;
+  return n <= 45056 || n > 90112 ? 32 : 64;
+}
+
 }  // namespace fo

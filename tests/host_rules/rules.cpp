@@ -38,6 +38,10 @@ int main() {
       in >> batch >> in_f >> hidden >> split;
       const char* names[] = {"thread", "split", "rows"};
       std::printf("%s\n", names[(int)fo::mlp_form(batch, in_f, hidden, split != 0)]);
+    } else if (rule == "gemv") {
+      int64_t n, k;
+      in >> n >> k;
+      std::printf("%d\n", fo::gemv_cells(n, k));
     } else {
       return 1;
     }

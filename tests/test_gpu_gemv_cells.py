@@ -1,4 +1,4 @@
-"""The GEMV's two block sizes (16 cells up to 4096 rows, 32 past them) around their last blocks, stages of 96
+"""The GEMV's block sizes (16 cells up to 4096 rows, 32 or 64 past them) around their last blocks, stages of 96
 elements and the load ring's rounds, with a strided output: bit for bit against the oracle's serial fold."""
 import numpy as np
 import pytest
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 F32, BF16 = fh.F32, fh.BF16
 
 
-@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 4095, 4096, 4097, 4128, 4129])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 4095, 4096, 4097, 4128, 4129, 8193, 8255, 8256, 8257, 16385])
 @pytest.mark.parametrize("k", [8, 96, 104, 392])
 @pytest.mark.parametrize("out_t", [F32, BF16])
 def test_gemv_cells_exact(rt, n, k, out_t):

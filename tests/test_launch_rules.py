@@ -92,3 +92,12 @@ def test_gemm_any_tile(ask, shape, tile):
     ("2049 73 23 0", "rows"), ("64 784 128 0", "rows")])
 def test_mlp_form(ask, shape, form):
     assert ask([f"mlp {shape}"]) == [form]
+
+
+# rows, K -> cells a block. Every N past 4096 took 32 once: 16384 x 4096, 32768 and 65536 rows were slower than on 64.
+@pytest.mark.parametrize("shape, cells", [
+    ("4096 1024", 16), ("4097 1024", 32), ("8192 4096", 32), ("8193 1024", 64), ("16384 4096", 64), ("16385 1024", 32),
+    ("24576 3584", 32), ("24576 3592", 64), ("24577 1024", 64), ("32768 200", 64), ("32769 1024", 32), ("45056 2048", 32),
+    ("45057 1024", 64), ("65536 200", 64), ("90112 1024", 64), ("155648 1024", 32), ("155648 760", 64)])
+def test_gemv_cells(ask, shape, cells):
+    assert ask([f"gemv {shape}"]) == [str(cells)]
