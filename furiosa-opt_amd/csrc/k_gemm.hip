@@ -1152,7 +1152,7 @@ void gemm_any_launch(hipStream_t s, const GemmDesc& d, const GemmWorkspace& ws, 
     const char* e = getenv("FO_GEMM_TILE");
     return e ? atoi(e) : 0;
   }();
-  if ((forced ? forced : gemm_any_tile(d.M, d.N, d.batch)) == 64)
+  if ((forced ? forced : gemm_any_tile(d.M, d.N, d.K, d.batch, KIND == kI8)) == 64)
     return gemm_launch_cfg<KIND, OUT, 64, 64, 2, 2, 2, false>(s, d, c, a, b, nullptr, nullptr,
                                                               splits_of(tiles_of(d, 64), d.K * MfmaT<KIND>::EB, 64), &ws);
   gemm_launch_cfg<KIND, OUT, 128, 128, 2, 2, 2, false>(s, d, c, a, b, nullptr, nullptr);
@@ -1220,7 +1220,7 @@ void launch_gemm(hipStream_t s, void* c, const void* a, const void* b, fo_dtype 
 bool launch_gemm_any(hipStream_t s, void* c, const void* a, const void* b, fo_dtype in_t, fo_dtype out_t,
                      const GemmDesc& d, const GemmWorkspace& ws) {
   if (d.M < 8 || d.N < 8 || d.K <= 0 || d.M >= (1ll << 31) || d.N >= (1ll << 31) || d.batch <= 0 || d.batch >= 65536) return false;
-  if (gemm_any_tile(d.M, d.N, d.batch) == 0) return false;
+  if (gemm_any_tile(d.M, d.N, d.K, d.batch, in_t == FO_I8) == 0) return false;
   if (d.K * 2 >= (1ll << 31) || 128 * std::max(d.lda, d.ldb) * 2 >= (1ll << 32)) return false;  // 32-bit offsets in a tile
   if (in_t == FO_BF16 && out_t == FO_BF16) return gemm_any_launch<kBf16, 0>(s, d, ws, c, a, b), true;
   if (in_t == FO_BF16 && out_t == FO_F32) return gemm_any_launch<kBf16, 1>(s, d, ws, c, a, b), true;

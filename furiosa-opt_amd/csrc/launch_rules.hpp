@@ -93,9 +93,31 @@ inline GemmTile gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, int el
 
 // Operands whose rows or K are off 16 bytes: 64x64 or 128x128 tiles staged through registers. As above, a
 // side of up to 64 keeps the smaller tile at any number of tiles (2000 x 32, 32, 63: 12.8 us against 28 bf16,
-// 14.1 against 34 i8, and 17-18 for the vector-unit fold that took it before). 0: no launch holds the tiles.
-inline int gemm_any_tile(int64_t m, int64_t n, int64_t batch) {
+// 14.1 against 34 i8, and 17-18 for the vector-unit fold that took it before). 0: the vector-unit fold, for what no
+// launch of these tiles holds and for a K so short that the tiles' fixed 4 us (i8: 5) are not paid back. Kernel
+// alone in a recorded graph, one box, us, fold / tiles:
+//     batch x M, N           K = 2         7            14           20           31           47
+//     i8    1 x 8, 8       2.8 / 4.7    3.0 / 4.7    3.2 / 4.7    3.4 / 4.9    3.7 / 4.8    4.7 / 4.9
+//     i8    1 x 100, 100   3.5 / 4.9    3.8 / 4.9    4.0 / 4.8    4.1 / 5.1    4.5 / 5.1    5.5 / 5.1
+//     i8    1 x 500, 500   4.0 / 5.1    4.3 / 5.1    4.5 / 5.1    4.7 / 5.3    5.1 / 5.3    6.2 / 5.3
+//     i8    1 x 700, 700   4.5 / 5.3    4.8 / 5.2    5.2 / 5.2    5.4 / 5.5    5.8 / 5.5    7.1 / 5.5
+//     i8    1000 x 16, 16  5.4 / 6.8    5.8 / 6.8    6.3 / 7.0    6.7 / 6.9    7.6 / 7.6   10.0 / 7.6
+//     i8    5000 x 8, 8     12 / 24      13 / 24      15 / 24      16 / 25      19 / 26      26 / 27
+//     i8    1 x 8, 30000   5.7 / 5.3    6.2 / 5.4    6.7 / 5.4    7.2 / 5.5    8.0 / 5.6   10.5 / 5.6
+//     bf16  1 x 8, 8       3.2 / 3.8    3.4 / 3.9    3.7 / 4.0    3.8 / 3.9    4.2 / 4.1    5.5 / 4.2
+//     bf16  1 x 100, 100   3.9 / 4.3    4.2 / 4.3    4.5 / 4.4    4.6 / 4.5    5.1 / 4.5    6.4 / 4.6
+//     bf16  1 x 500, 500   4.3 / 4.5    4.6 / 4.5    4.9 / 4.6    5.2 / 4.7    5.7 / 4.7    6.9 / 4.8
+//     bf16  5000 x 8, 8     15 / 19      16 / 19      18 / 19      19 / 19      22 / 21      30 / 23
+inline int64_t gemm_any_min_k(int64_t m, int64_t n, int64_t batch, bool i8) {
+  const int64_t cells = m * n * batch;
+  if (cells <= 128 * tiles_of(m, n, batch, 64, 64)) return i8 ? 48 : 20;  // tiles nearly empty
+  if (!i8) return cells <= (1 << 17) ? 8 : 0;
+  if (std::min(m, n) < 16) return cells <= (1 << 16) ? 32 : 0;
+  return cells <= (1 << 18) ? 32 : cells <= (1 << 19) ? 16 : 0;
+}
+inline int gemm_any_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool i8) {
   auto fits = [&](int64_t t) { return tiles_of(m, n, 1, t, t) * 256 < (1ll << 32); };
+  if (k < gemm_any_min_k(m, n, batch, i8)) return 0;
   if ((tiles_of(m, n, batch, 64, 64) <= 512 || std::min(m, n) <= 64) && fits(64)) return 64;
   return fits(128) ? 128 : 0;
 }

@@ -29,9 +29,10 @@ int main() {
       in >> type >> batch >> m >> n >> k;
       std::printf("%d\n", (int)fo::gemm_tile(m, n, k, batch, type == "bf16" ? 2 : 1, type == "f8"));
     } else if (rule == "gemm_any") {
-      int64_t batch, m, n;
-      in >> batch >> m >> n;
-      std::printf("%d\n", fo::gemm_any_tile(m, n, batch));
+      std::string type;
+      int64_t batch, m, n, k;
+      in >> type >> batch >> m >> n >> k;
+      std::printf("%d\n", fo::gemm_any_tile(m, n, k, batch, type == "i8"));
     } else if (rule == "mlp") {
       int64_t batch, in_f, hidden;
       int split;

@@ -71,10 +71,16 @@ def test_gemm_tile(ask, shape, tile):
     assert ask([f"gemm {shape}"]) == [str(tile)]
 
 
-# batch, m, n -> tile of the contraction off 16-byte rows; batches of small products went to 128x128 once
-@pytest.mark.parametrize("shape, tile", [("1 333 1000", 64), ("1 1500 2000", 128), ("2000 32 32", 64), ("600 64 200", 64), ("600 65 70", 128),
-                                         ("1 16 155648", 64), ("1 8 1073741760", 64), ("1 8 1073741888", 128),
-                                         ("1 8 2147483647", 0)])
+# type, batch, m, n, k -> tile of the contraction off 16-byte rows (0: the vector-unit fold). Batches of small products
+# went to 128x128 once, and a K too short for the tiles to them: i8 8 x 8 x 31 4.8 us against 3.7.
+@pytest.mark.parametrize("shape, tile", [
+    ("bf16 1 333 1000 777", 64), ("bf16 1 1500 2000 71", 128), ("i8 2000 32 32 63", 64), ("bf16 600 64 200 63", 64),
+    ("bf16 600 65 70 63", 128), ("bf16 1 16 155648 129", 64), ("i8 1 8 1073741760 63", 64), ("i8 1 8 1073741888 63", 128),
+    ("i8 1 8 2147483647 63", 0),
+    ("i8 1 8 8 47", 0), ("i8 1 8 8 49", 64), ("bf16 1 8 8 19", 0), ("bf16 1 8 8 21", 64), ("i8 5000 8 8 47", 0),
+    ("i8 1 500 500 31", 0), ("i8 1 500 500 33", 64), ("i8 1 700 700 15", 0), ("i8 1 700 700 17", 64), ("i8 1 1000 1000 2", 64),
+    ("i8 1 9 3000 31", 0), ("i8 1 8 30000 2", 64), ("i8 1000 16 16 17", 0), ("bf16 1 100 100 7", 0), ("bf16 1 100 100 9", 64),
+    ("bf16 1 500 500 2", 64), ("bf16 1 333 1000 7", 64)])
 def test_gemm_any_tile(ask, shape, tile):
     assert ask([f"gemm_any {shape}"]) == [str(tile)]
 
