@@ -8,7 +8,7 @@
 // wave's load or store is 1 KiB contiguous. exp(y - max) is held in f32 registers from the sum to the
 // output, so each element is read, exponentiated and written once. Two kernels:
 //   * k_rmsnorm_softmax_row (up to 32768 columns, any row length): one to sixteen waves per row;
-//   * k_rmsnorm_softmax_dma (4096 columns, many rows): one wave per row, persistent waves, the next row
+//   * k_rmsnorm_softmax_dma (2048 or 4096 columns, many rows): one wave per row, persistent waves, the next row
 //     fetched into LDS by DMA while the current one is computed, the gain staged once per block.
 // Bound by HBM when large (5.1-5.4 TB/s, what a large copy reaches) and by the launch and one memory
 // round trip when small.
@@ -19,7 +19,7 @@
 // subnormal reads as zero in every later op), a subnormal result flushes before the narrow, and
 // the narrow is the hardware round-to-nearest-even v_cvt_pk_bf16_f32. The one case left is a
 // non-finite value (NaN payloads and inf - inf), which the reference canonicalises: a row whose
-// sum of squares is non-finite, whose mean square is not positive (a division by zero) or whose gain
+// sum of squares is non-finite, whose mean square may not be positive (a division by zero) or whose gain
 // reaches kGainMax is computed by the exact per-element path.
 //   * (x*g)/r is the correctly rounded quotient q' = RN(q + e*y), q = RN(a*y), e = a - q*r (exact,
 //     one FMA), y = RN(1/r) (Markstein's correction, exact for normal operands and results);
@@ -129,7 +129,7 @@ __device__ void row_exact(uint16_t* __restrict__ orow, const uint16_t* __restric
   }
 }
 
-// Rows of 4096 columns: one wave per row, persistent waves, the next row fetched into LDS
+// Rows of 2048 or 4096 columns: one wave per row, persistent waves, the next row fetched into LDS
 // by DMA (buffer_load ... lds) while the current one is computed. A register prefetch would not
 // stay in flight: with this row's stores also outstanding the compiler waits for every access
 // before touching the prefetched registers. Here the only wait on vector memory is explicit and
@@ -184,6 +184,9 @@ __global__ void __launch_bounds__(64 * kDmaWaves) k_rmsnorm_softmax_dma(uint16_t
   __syncthreads();
   const bool gain_bad = __syncthreads_or(bad_local) != 0;
   if (row >= rows) return;
+  // Sums of squares from here on have a positive mean square: with an eps every one, without it those that the
+  // division can't flush. Comparing the sum itself keeps the division off the branch (8000 x 2048: 13.6 us with it).
+  const float ss_min = gain_bad ? INFINITY : eps >= 0x1p-126f ? 0.f : eps >= 0.f ? 0x1p-100f : INFINITY;
   __builtin_amdgcn_s_waitcnt(waitcnt_vm0);
 
   for (; row < rows; row += nwaves) {
@@ -207,12 +210,12 @@ __global__ void __launch_bounds__(64 * kDmaWaves) k_rmsnorm_softmax_dma(uint16_t
     }
     const float ss = wave_sum(ss0 + ss1);
     uint16_t* orow = out + row * cols;
-    const float ms = __fadd_rn(__fdiv_rn(ss, cols_f), eps);  // fp_div, then clip Add eps
-    if (!__builtin_isfinite(ss) || !(ms > 0.f) || gain_bad) {
+    if (!(ss >= ss_min && ss < INFINITY)) {
       row_exact(orow, x + row * cols, gain, cols, eps, lane);
       __builtin_amdgcn_s_waitcnt(waitcnt_vm0);
       continue;
     }
+    const float ms = __fadd_rn(__fdiv_rn(ss, cols_f), eps);  // fp_div, then clip Add eps
     const float r = sqrt_rn(ms);                              // FpUnaryOp::Sqrt
     const float rinv = __fdiv_rn(1.0f, r);
     // y = bf16((x * g) / r), kept packed; row max on the f32 values
@@ -443,17 +446,16 @@ void launch_rmsnorm_softmax(hipStream_t s, uint16_t* out, const uint16_t* x, con
   // the per-element path that took every column count the DMA form does not):
   //     rows, cols     row kernel   before        rows, cols     row kernel   before
   //     500, 512          3.1     4.4 (DMA)       500, 3072         4.5     41 (exact)
-  //     32768, 1024      24.4    26.2 (DMA)       8192, 4096       26.8     25.7 (DMA)
+  //     32768, 1024      24.4    26.2 (DMA)
   //     500, 4096         4.5    12.2 (DMA)       4096, 8192       28.7     30.8 (rows split over 4 waves)
-  // so the DMA form is kept where it is the faster one, past 6144 rows of 4096 (15.3 against 16.0 at 4096
-  // rows). W and P are the best of one to sixteen waves a row; wider rows want more waves while the
+  // The DMA form is kept where it is the faster one (norm_dma). W and P are the best of one to sixteen waves a row; wider rows want more waves while the
   // result is small (2048 columns: 3.7 us with 4 waves against 3.9 with 2 at 500 rows; 32.4 against 26.2 at
   // 16384). Past 10 MiB a tensor the accesses stream past the caches (1500, 4096: 7.9 against 9.1 us;
   // at 4 MiB 5.3 against 4.5).
   const bool aligned = (((uintptr_t)x | (uintptr_t)out | (uintptr_t)gain) & 15) == 0;
   const bool stream = rows * cols * 2 >= (10ll << 20);
-  if (aligned && cols == 4096 && rows >= 6144) {
-    rs_dma_launch<8>(s, out, x, gain, rows, eps);
+  if (aligned && norm_dma(rows, cols)) {
+    cols == 4096 ? rs_dma_launch<8>(s, out, x, gain, rows, eps) : rs_dma_launch<4>(s, out, x, gain, rows, eps);
   } else if (cols <= 32768) {
     if (cols <= 512)
       rs_row_launch<8, 1>(s, out, x, gain, rows, cols, eps, stream);

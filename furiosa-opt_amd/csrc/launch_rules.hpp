@@ -16,6 +16,21 @@ void for_row_pieces(int64_t rows, int64_t threads_per_row, F&& f) {
   for (int64_t first = 0; first < rows; first += per) f(first, std::min(per, rows - first));
 }
 
+// RMSNorm -> softmax of aligned rows: whether the persistent DMA form (k_rmsnorm_softmax_dma, 4096 rows a round of
+// the chip) takes them from the row kernel. It hides a round's loads behind the last one's work but pays a whole
+// round for a part of one. Kernel alone in a recorded graph, one box, us, DMA / row kernel:
+//     rows         3500          4000          4096          4500          6000          8000          8192
+//     2048      8.2 / 6.7     8.3 / 7.1     8.3 / 7.1    11.6 / 7.9    11.6 / 10.1   12.5 / 13.3   12.8 / 13.4
+//     4096     14.0 / 12.9   12.8 / 14.2   12.8 / 14.5   19.9 / 15.1   22.0 / 19.4       -         25.7 / 26.8
+//     rows         9000         11000         12288         14000         16384         20000         32768
+//     2048     16.2 / 14.2   17.9 / 17.1   18.6 / 19.2   23.4 / 21.6   25.6 / 26.8   30.2 / 31.7   48.7 / 49.7
+// and of 1024 columns and fewer the row kernel is the faster one at every number of rows.
+inline bool norm_dma(int64_t rows, int64_t cols) {
+  const int64_t last = (rows - 1) % 4096 + 1;  // rows of the last round
+  if (cols == 4096) return rows >= 6144 || (rows > 3840 && rows <= 4096);
+  return cols == 2048 && rows > 4096 && rows <= 32768 && last > 3400;
+}
+
 // Attention without a given row max: 2 groups of 32 queries x 4 of keys a workgroup, 4 x 2, or 256 queries.
 // By the workgroups each would have (WG64 and WG128: one per 64 or 128 queries of a head). Kernel alone in
 // a recorded graph, D = 128, us (one box), causal / not:

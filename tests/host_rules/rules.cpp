@@ -43,6 +43,10 @@ int main() {
       int64_t n, k;
       in >> n >> k;
       std::printf("%d\n", fo::gemv_cells(n, k));
+    } else if (rule == "norm") {
+      int64_t rows, cols;
+      in >> rows >> cols;
+      std::printf("%s\n", fo::norm_dma(rows, cols) ? "dma" : "row");
     } else {
       return 1;
     }

@@ -12,7 +12,9 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(3, 1), (5, 7), (9, 8), (6, 63), (5, 511), (5, 513), (7, 1001), (3, 1024), (5, 1025), (3, 2047), (2, 2049),
           (3, 4095), (2, 4097), (3, 8191), (2, 8193), (2, 16383), (1, 16385), (2, 32767), (1, 32768), (1, 32769),
           # past 10 MiB a tensor: streamed accesses, two waves a row up to 3072 columns
-          (5200, 1025), (3000, 2047), (2601, 2049), (1710, 3072), (1706, 3073), (6144, 4096)]
+          (5200, 1025), (3000, 2047), (2601, 2049), (1710, 3072), (1706, 3073), (6144, 4096),
+          # the DMA form at 2048 columns, whole and partial last rounds, and one round of 4096
+          (7497, 2048), (8192, 2048), (4096, 4096), (3841, 4096)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))

@@ -107,3 +107,13 @@ def test_mlp_form(ask, shape, form):
     ("45057 1024", 64), ("65536 200", 64), ("90112 1024", 64), ("155648 1024", 32), ("155648 760", 64)])
 def test_gemv_cells(ask, shape, cells):
     assert ask([f"gemv {shape}"]) == [str(cells)]
+
+
+# rows, columns -> form. The row kernel took every number of rows of 2048 columns, and 4096 rows of 4096, once.
+@pytest.mark.parametrize("shape, form", [
+    ("8192 4096", "dma"), ("6144 4096", "dma"), ("6143 4096", "row"), ("4097 4096", "row"), ("4096 4096", "dma"),
+    ("3840 4096", "row"), ("8192 2048", "dma"), ("8193 2048", "row"), ("7496 2048", "row"), ("7497 2048", "dma"),
+    ("4096 2048", "row"), ("20000 2048", "dma"), ("32768 2048", "dma"), ("36864 2048", "row"), ("8192 1024", "row"),
+    ("8192 2047", "row")])
+def test_norm_form(ask, shape, form):
+    assert ask([f"norm {shape}"]) == [form]
