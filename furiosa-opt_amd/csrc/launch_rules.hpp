@@ -65,8 +65,13 @@ inline AttnForm attention_form(int64_t heads, int64_t seq, bool causal) {
 //     bf16  1024, 4096, 512         13.1        10.4               10.0             20      8 stages of 128 bytes of k
 //     bf16  343, 5584, 384           9.7         8.6                8.2             26      6
 //     i8    900, 3500, 1024         13.7        11.5               11.2             24      8
-//     i8    1024, 4096, 1536         -          14.1               14.4              -      12
-//     bf16  1024, 4096, 1536         -          18.5               22.4              -      24
+//     i8    1024, 3000, 1536         -          12.9               12.2              -      12
+//     bf16  640, 4096, 768           -          10.0                9.6              -      12
+//     f8    900, 3000, 1536          -          11.1               12.3              -      12
+//     bf16  640, 4096, 1024          -          11.4               11.1              -      16
+//     i8    777, 4096, 2048          -          13.4               13.4              -      16
+//     i8    900, 4096, 2560          -          16.7               18.0              -      20
+//     bf16  1024, 3000, 1280         -          14.1               15.8              -      20
 //     bf16  2048, 4096, 4096       104          75.0               66.9             80      T128 = 512, T256 = 128
 //     f8    2048, 4096, 4096        58          45.7               36.6             52
 //     bf16  1500, 5500, 1024        37.9        39.9               35.2             44      T128 = 516, T256 = 132
@@ -100,7 +105,7 @@ inline GemmTile gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, int el
   auto fits = [&](int64_t tm, int64_t tn, int64_t threads) { return tiles_of(m, n, 1, tm, tn) * threads < (1ll << 32); };
   if (m <= 32 && fits(32, 64, 128)) return kTile32x64;
   if ((t64 <= 512 || side <= 64) && fits(64, 64, 256)) return kTile64;
-  if (t128 <= 256 && (k * elem_bytes + 127) / 128 >= 12) return kTile128Deep;
+  if (t128 <= 256 && (k * elem_bytes + 127) / 128 >= (f8 ? 12 : 18)) return kTile128Deep;
   if ((t128 <= 512 || side <= 128) && fits(128, 128, 256)) return kTile128;
   if (tiles_of(m, n, batch, 256, 256) < 144 && k <= (f8 ? 512 : 1024)) return kTile128;
   return kTile256;

@@ -40,7 +40,7 @@ def product(a, b):
 # stages in flight among them, and small sides past 512 tiles.
 SIZES = [(8, 8, 16), (64, 64, 64), (65, 63, 80), (9, 70, 6160), (64, 64, 12304), (130, 200, 4624), (128, 1030, 2080),
          (257, 8136, 512), (520, 4096, 144), (2048, 2049, 96), (2300, 4090, 64), (3072, 3000, 48),
-         (257, 8136, 1552), (20, 33000, 80), (33010, 63, 48), (33000, 40, 272), (70, 70000, 48)]
+         (257, 8136, 1552), (257, 8136, 2320), (20, 33000, 80), (33010, 63, 48), (33000, 40, 272), (70, 70000, 48)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
