@@ -278,7 +278,7 @@ __global__ void __launch_bounds__(kMlpThreads) k_mlp_split(int32_t* __restrict__
 // ascending, the emulator's own fold. Weights go through LDS as bf16 bits (subnormals already read as
 // zero), 32 k at a time, double-buffered, the 16-byte loads (any address) of the next two chunks in
 // flight; each weight is read once per block instead of once per row. Bound by the multiplies and adds
-// when RT is large (4096 x 784 x 128: 45 us against 21 us of them on every SIMD), by each chunk's chain of
+// when RT is large (4096 x 784 x 128: 42 us against 21 us of them on every SIMD), by each chunk's chain of
 // LDS reads, serial adds, LDS writes and barrier (0.53 us) when it is 1.
 constexpr int kRowsT = 512;      // threads
 constexpr int kRowsKC = 32;      // k per chunk

@@ -9,8 +9,8 @@ from test_gpu_gemm_tiles import TYPES, narrowed, operands, product
 
 pytestmark = pytest.mark.gpu
 
-# K below a chunk, around a stage (64 bf16, 128 i8), prefetch depths, shared tiles with an uneven last
-# run, and the larger tile; rows past the last tile.
+# K below a chunk (small outputs of it go to the vector-unit fold, 1000 x 777 x 2 to the tiles), around a stage
+# (64 bf16, 128 i8), prefetch depths, shared tiles with an uneven last run, and the larger tile; rows past the last tile.
 SIZES = [(8, 8, 1), (8, 9, 7), (65, 64, 63), (64, 65, 65), (70, 33, 127), (33, 70, 129), (64, 64, 255), (9, 100, 321),
          (40, 24, 6145), (128, 200, 3331), (333, 1000, 777), (2113, 1100, 71), (1500, 2000, 131),
          # either side of the shortest K that the tiles take
