@@ -110,6 +110,7 @@ struct GemmArgs {
   int64_t a_batch, b_batch, c_batch;
   int32_t tiles_m, tiles_n;
   int32_t splits;      // blocks sharing an output tile, each a run of k stages (k_gemm; 1: none)
+  uint32_t per_split;  // splits > 1: 2^32 / splits, rounded up
   uint64_t* parts;     // splits > 1: partial accumulators
   uint32_t* arrived;   // splits > 1: blocks of each tile that have stored theirs (zero between launches)
   const float* scale;  // OUT == 4: per-column dequant scale
@@ -271,13 +272,10 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   // contiguous range of tiles, ordered in groups of 8 tile-rows so neighbours share operands in L2.
   const int ntiles = g.tiles_m * g.tiles_n;
   // Blocks share tiles only of the smaller sizes (splits_of); the others carry no code for it (0.3-0.5 us
-  // a launch: f8 1000 x 8 x 8 x 64 13.1 us against 14.0).
+  // a launch: f8 1000 x 8 x 8 x 64 13.1 us against 14.0). The block's share is a dimension of the grid and its
+  // stages come by multiplication: dividing for either cost a shared launch another 0.3-0.5 us.
   constexpr bool SHARED = BM <= 64 && BN <= 64;
-  int split = 0, bid = blockIdx.x;
-  if (SHARED && g.splits > 1) {  // uniform
-    split = bid / ntiles;
-    bid -= split * ntiles;
-  }
+  const int split = SHARED ? blockIdx.z : 0, bid = blockIdx.x;
   int tile = bid;
   if ((ntiles % 8) == 0) tile = (bid % 8) * (ntiles / 8) + bid / 8;
   const int group = 8;
@@ -297,9 +295,9 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   const uint32_t KB = (uint32_t)(g.K * EB);  // K in bytes
   // This block's k stages: [st0, st0 + nst) of the contraction's.
   int st0 = 0, nst = (int)((KB + kRB - 1) / kRB);
-  if (SHARED && g.splits > 1) {  // at most 8 splits of fewer than 2^24 stages
-    const int end = nst * (split + 1) / g.splits;
-    st0 = nst * split / g.splits;
+  if (SHARED && g.splits > 1) {  // uniform; x / splits = x * per_split >> 32 for x < 2^29: 8 splits of 2^24 stages
+    const int end = (int)__umulhi((uint32_t)(nst * (split + 1)), g.per_split);
+    st0 = (int)__umulhi((uint32_t)(nst * split), g.per_split);
     nst = end - st0;
   }
 
@@ -1065,6 +1063,7 @@ GemmArgs gemm_args(const GemmDesc& d, void* c, const void* a, const void* b, con
   g.b_batch = d.b_batch;
   g.c_batch = d.c_batch;
   g.splits = 1;
+  g.per_split = 0;
   g.parts = nullptr;
   g.arrived = nullptr;
   g.scale = scale;
@@ -1098,6 +1097,7 @@ void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, c
   require(splits == 1 || (BM <= 64 && BN <= 64), "gemm: blocks share tiles of up to 64x64 only");
   if (splits > 1) {
     g.splits = splits;
+    g.per_split = (uint32_t)(((1ull << 32) + splits - 1) / splits);
     g.parts = ws->parts;
     g.arrived = ws->arrived;
   }
@@ -1108,7 +1108,7 @@ void gemm_launch_cfg(hipStream_t s, const GemmDesc& d, void* c, const void* a, c
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_set = true;
   }
-  dim3 grid((unsigned)(tiles * splits), (unsigned)d.batch);
+  dim3 grid((unsigned)tiles, (unsigned)d.batch, (unsigned)splits);
   hipLaunchKernelGGL((k_gemm<KIND, OUT, BM, BN, WM, WN, NS, DMA>), grid, dim3(64 * WM * WN), lds, s, g);
   FO_HIP(hipGetLastError());
 }
