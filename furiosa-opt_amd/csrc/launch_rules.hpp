@@ -62,16 +62,6 @@ inline AttnForm attention_form(int64_t heads, int64_t seq, bool causal) {
 //     bf16  500, 3072, 1024         10.0        12.9               15.3             38
 //     bf16  512, 4096, 4096         30.7        32.3               42.6             75      T64 = 512
 //     bf16  1024, 4096, 4096        58          39.3               48.6             76      T128 = 256
-//     bf16  1024, 4096, 512         13.1        10.4               10.0             20      8 stages of 128 bytes of k
-//     bf16  343, 5584, 384           9.7         8.6                8.2             26      6
-//     i8    900, 3500, 1024         13.7        11.5               11.2             24      8
-//     i8    1024, 3000, 1536         -          12.9               12.2              -      12
-//     bf16  640, 4096, 768           -          10.0                9.6              -      12
-//     f8    900, 3000, 1536          -          11.1               12.3              -      12
-//     bf16  640, 4096, 1024          -          11.4               11.1              -      16
-//     i8    777, 4096, 2048          -          13.4               13.4              -      16
-//     i8    900, 4096, 2560          -          16.7               18.0              -      20
-//     bf16  1024, 3000, 1280         -          14.1               15.8              -      20
 //     bf16  2048, 4096, 4096       104          75.0               66.9             80      T128 = 512, T256 = 128
 //     f8    2048, 4096, 4096        58          45.7               36.6             52
 //     bf16  1500, 5500, 1024        37.9        39.9               35.2             44      T128 = 516, T256 = 132
@@ -82,7 +72,7 @@ inline AttnForm attention_form(int64_t heads, int64_t seq, bool causal) {
 //     f8    1500, 5500, 2048        34.9        39.4               35.0             32.0
 //     bf16  2048, 8192, 1024        68          54                 44.8             37.5    T256 = 256
 // Hence: 64x64 (32 KiB of LDS a stage pair, two blocks a CU) up to two tiles a CU; 128x128 with four stages
-// in flight while one block a CU covers them and K has stages enough to pay for filling four; with two
+// in flight while one block a CU covers them and K has stages enough to pay for filling four (deep_stages); with two
 // stages, two blocks a CU, up to 512; past that 256x256, but for the first, mostly empty round of them over a short K (1024 elements; 512 of the 8-bit
 // floats, whose 256x256 form is the faster one). An output side of up to 32, 64 or 128 keeps the tile as small
 // at any number of tiles, the rest of a larger one being padding (batch x M, N, K):
@@ -95,9 +85,29 @@ inline AttnForm attention_form(int64_t heads, int64_t seq, bool causal) {
 //     bf16  520 x 16, 64, 256        5.8    7.7         11.2           34.2
 //     f8    600 x 64, 64, 512        -     10.9         16.0           27.3
 //     bf16  300 x 100, 100, 256      -     16.3         10.7           45.3
+//
+// Stages of k from which 128x128 tiles keep four in flight, not two. A number of tiles that the 8 XCDs don't divide
+// is walked in launch order, neighbours on different XCDs' caches, and waits longer for each stage. us, two / four,
+// by stages of 128 bytes of k:
+//     types, M, N (tiles)         5            7            9           11           13           15           17
+//     bf16  777, 4096 (224)   7.1 / 7.4    7.9 / 8.4    8.7 / 9.2    9.5 / 9.9   10.2 / 10.6  11.0 / 11.3  11.9 / 12.2
+//     bf16  1024, 3000 (192)  7.3 / 7.7    8.2 / 8.7    9.0 / 9.4    9.7 / 10.2  10.5 / 10.8  11.6 / 11.5  12.9 / 12.3
+//       K off 128 bytes       7.5 / 7.9    8.4 / 8.8    9.3 / 9.4   10.3 / 10.2  11.4 / 11.1  12.4 / 11.7  13.8 / 12.6
+//     i8    777, 4096 (224)   8.1 / 8.4    8.9 / 9.5    9.8 / 10.2  10.6 / 11.0  11.3 / 11.7  12.2 / 12.4  14.3 / 13.5
+//     i8    900, 3000 (192)   8.0 / 8.6    8.9 / 9.4    9.8 / 10.1  10.9 / 10.9  11.9 / 11.7  13.2 / 12.3  14.4 / 13.2
+//     f8    900, 3000 (192)   7.9 / 8.2    8.8 / 9.1    9.7 / 9.8   10.9 / 10.6  12.1 / 11.6  13.5 / 12.3  14.8 / 13.2
+//     bf16  583, 5384 (215)   8.4 / 8.6    9.2 / 9.2   11.3 / 10.3  13.2 / 11.8  14.8 / 13.2  16.3 / 14.4  17.8 / 15.8
+//     bf16  343, 5584 (132)   7.1 / 7.4    7.9 / 8.5    8.8 / 9.2   11.1 / 10.1  12.5 / 10.8  14.7 / 11.8  16.2 / 12.5
+//       K off 128 bytes       7.2 / 7.5    8.1 / 8.4   10.0 / 9.5   10.7 / 10.3  14.1 / 12.0  15.8 / 13.1  17.4 / 14.4
+//     i8    640, 3300 (130)   8.1 / 8.3    9.5 / 9.6   10.7 / 10.4  12.2 / 11.3  14.2 / 12.1  16.0 / 12.9  17.4 / 13.8
+//     f8    583, 5384 (215)   9.1 / 9.1   10.5 / 10.1  12.4 / 11.1  14.3 / 12.4  16.0 / 13.8  17.5 / 14.8  19.1 / 16.1
 enum GemmTile { kTile32x64 = 32, kTile64 = 64, kTile128 = 128, kTile128Deep = 1284, kTile256 = 256 };
 inline int64_t tiles_of(int64_t m, int64_t n, int64_t batch, int64_t tm, int64_t tn) {
   return ((m + tm - 1) / tm) * ((n + tn - 1) / tn) * batch;
+}
+inline int64_t deep_stages(int64_t tiles, int elem_bytes, bool f8) {
+  if (tiles % 8) return elem_bytes == 2 ? 9 : 8;
+  return elem_bytes == 2 ? 15 : f8 ? 10 : 13;
 }
 inline GemmTile gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes, bool f8) {
   const int64_t t64 = tiles_of(m, n, batch, 64, 64), t128 = tiles_of(m, n, batch, 128, 128), side = std::min(m, n);
@@ -105,7 +115,7 @@ inline GemmTile gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, int el
   auto fits = [&](int64_t tm, int64_t tn, int64_t threads) { return tiles_of(m, n, 1, tm, tn) * threads < (1ll << 32); };
   if (m <= 32 && fits(32, 64, 128)) return kTile32x64;
   if ((t64 <= 512 || side <= 64) && fits(64, 64, 256)) return kTile64;
-  if (t128 <= 256 && (k * elem_bytes + 127) / 128 >= (f8 ? 12 : 18)) return kTile128Deep;
+  if (t128 <= 256 && (k * elem_bytes + 127) / 128 >= deep_stages(tiles_of(m, n, 1, 128, 128), elem_bytes, f8)) return kTile128Deep;
   if ((t128 <= 512 || side <= 128) && fits(128, 128, 256)) return kTile128;
   if (tiles_of(m, n, batch, 256, 256) < 144 && k <= (f8 ? 512 : 1024)) return kTile128;
   return kTile256;
