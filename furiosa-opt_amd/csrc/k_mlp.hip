@@ -501,7 +501,7 @@ void launch_mlp(hipStream_t s, int32_t* pred, uint16_t* logits, const uint16_t* 
   // graph, batch x inputs x hidden x outputs, us, a row a block -> k_mlp_rows:
   //     1024 x 784 x 128 x 10     46.7 (split) -> 26      1104 x 270 x 147 x 33    32.6 (k_mlp) -> 24
   //     4096 x 784 x 128 x 10    179.7 (split) -> 42      4096 x 1024 x 512 x 64    955 (k_mlp) -> 185
-  if (mlp_form(batch, in_f, hidden, split) == MlpForm::kRows) {
+  if (mlp_form(batch, in_f, hidden, out_f, split) == MlpForm::kRows) {
     MlpArgs g{pred, logits, x, w1, b1, w2, b2, (int32_t)batch, (int32_t)in_f, (int32_t)hidden, (int32_t)out_f, 0, 0, 0, 0};
     if (batch > 2048 && mlp_rows_launch<16>(s, g)) return;
     if (batch > 1024 && mlp_rows_launch<8>(s, g)) return;

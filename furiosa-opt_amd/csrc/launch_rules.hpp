@@ -180,16 +180,16 @@ inline int gemm_any_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool i8
 //     70, 200, 5               10.5 / 11.5    11.9 / 11.9       -             -           -           -
 //     195, 65, 10              11.9 / 10.1    12.6 / 10.6    14.1 / 11.4   14.0 / 12.2 19.6 / 12.6 21.0 / 12.7
 // k_mlp's time is its two serial folds, an input costing about two hidden values; k_mlp_rows pays about 0.55 us
-// a chunk of 32 of either.
+// a chunk of 32 of either, and more past 32 outputs (362 x 123 x 17 x 50 8.4 / 9.7; 512 x 130 x 130 x 50 13.4 / 14.1).
 enum class MlpForm { kThread, kSplit, kRows };
-inline MlpForm mlp_form(int64_t batch, int64_t in_f, int64_t hidden, bool split) {
+inline MlpForm mlp_form(int64_t batch, int64_t in_f, int64_t hidden, int64_t out_f, bool split) {
   if (split) {
     const bool wide = (hidden > 104 && hidden <= 128 && in_f >= 256) || hidden % 32 > 16;
     return batch <= (wide && hidden > 64 && hidden <= 128 ? 256 : 512) ? MlpForm::kSplit : MlpForm::kRows;
   }
   const int64_t folds = 2 * in_f + hidden;
   const bool thread = batch <= 256    ? folds <= 344 && hidden <= 256
-                      : batch <= 512  ? folds <= 240 && hidden <= 80
+                      : batch <= 512  ? (out_f > 32 ? folds <= 400 && hidden <= 130 : folds <= 240 && hidden <= 80)
                       : batch <= 1024 ? folds <= 315 && hidden <= 128
                                       : batch <= 2048 && folds <= 260 && hidden <= 64;
   return thread ? MlpForm::kThread : MlpForm::kRows;

@@ -34,11 +34,11 @@ int main() {
       in >> type >> batch >> m >> n >> k;
       std::printf("%d\n", fo::gemm_any_tile(m, n, k, batch, type == "i8"));
     } else if (rule == "mlp") {
-      int64_t batch, in_f, hidden;
+      int64_t batch, in_f, hidden, out_f;
       int split;
-      in >> batch >> in_f >> hidden >> split;
+      in >> batch >> in_f >> hidden >> out_f >> split;
       const char* names[] = {"thread", "split", "rows"};
-      std::printf("%s\n", names[(int)fo::mlp_form(batch, in_f, hidden, split != 0)]);
+      std::printf("%s\n", names[(int)fo::mlp_form(batch, in_f, hidden, out_f, split != 0)]);
     } else if (rule == "gemv") {
       int64_t n, k;
       in >> n >> k;

@@ -16,7 +16,8 @@ SHAPES = [(1, 31, 100, 2), (3, 129, 16, 64), (2, 100, 1024, 63), (5, 33, 513, 17
           (300, 1024, 20, 33), (512, 72, 64, 9), (513, 72, 64, 9), (257, 72, 65, 9), (1, 4000, 1024, 64), (7, 100, 28, 3),
           # both sides of the lines between the one-row forms and k_mlp_rows
           (3, 72, 200, 5), (3, 72, 201, 5), (257, 80, 80, 7), (257, 81, 79, 7), (400, 256, 128, 9), (512, 131, 65, 9),
-          (1000, 100, 100, 50), (600, 161, 33, 16), (1025, 100, 60, 10), (1500, 73, 90, 10), (2048, 73, 23, 34), (2049, 73, 23, 34)]
+          (1000, 100, 100, 50), (600, 161, 33, 16), (1025, 100, 60, 10), (1500, 73, 90, 10), (2048, 73, 23, 34), (2049, 73, 23, 34),
+          (362, 123, 17, 50), (300, 131, 131, 50)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))

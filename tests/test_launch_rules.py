@@ -87,17 +87,18 @@ def test_gemm_any_tile(ask, shape, tile):
     assert ask([f"gemm_any {shape}"]) == [str(tile)]
 
 
-# batch, inputs, hidden, whether k_mlp_split takes the shape -> form. The lines stood at in_f + hidden <= 128 up to
+# batch, inputs, hidden, outputs, whether k_mlp_split takes the shape -> form. The lines stood at in_f + hidden <= 128 up to
 # 256 rows (100 x 50 and 70 x 200 were slower on k_mlp_rows, all of k_mlp's past 256 rows) and, from 65 units, at
 # 256 rows of k_mlp_split (400 x 72, 1024 x 136).
 @pytest.mark.parametrize("shape, form", [
-    ("64 784 128 1", "split"), ("256 784 128 1", "split"), ("257 784 128 1", "rows"), ("257 248 128 1", "split"),
-    ("512 400 72 1", "split"), ("512 1024 104 1", "split"), ("257 256 105 1", "rows"), ("512 1024 136 1", "split"), ("257 64 88 1", "rows"), ("512 64 56 1", "split"),
-    ("513 64 16 1", "rows"), ("513 1024 136 1", "rows"),
-    ("1 73 23 0", "thread"), ("256 100 50 0", "thread"), ("1 70 200 0", "thread"), ("64 72 201 0", "rows"), ("64 30 257 0", "rows"),
-    ("257 73 23 0", "thread"), ("512 95 50 0", "thread"), ("512 96 50 0", "rows"), ("320 30 90 0", "rows"), ("513 105 105 0", "thread"),
-    ("1024 30 129 0", "rows"), ("1025 100 60 0", "thread"), ("1025 75 75 0", "rows"), ("2048 73 23 0", "thread"),
-    ("2049 73 23 0", "rows"), ("64 784 128 0", "rows")])
+    ("64 784 128 10 1", "split"), ("256 784 128 10 1", "split"), ("257 784 128 10 1", "rows"), ("257 248 128 10 1", "split"),
+    ("512 400 72 10 1", "split"), ("512 1024 104 10 1", "split"), ("257 256 105 10 1", "rows"), ("512 1024 136 10 1", "split"), ("257 64 88 10 1", "rows"), ("512 64 56 10 1", "split"),
+    ("513 64 16 10 1", "rows"), ("513 1024 136 10 1", "rows"),
+    ("1 73 23 10 0", "thread"), ("256 100 50 10 0", "thread"), ("1 70 200 10 0", "thread"), ("64 72 201 10 0", "rows"), ("64 30 257 10 0", "rows"),
+    ("257 73 23 10 0", "thread"), ("512 95 50 10 0", "thread"), ("512 96 50 10 0", "rows"), ("320 30 90 10 0", "rows"), ("513 105 105 10 0", "thread"),
+    ("1024 30 129 10 0", "rows"), ("1025 100 60 10 0", "thread"), ("1025 75 75 10 0", "rows"), ("2048 73 23 10 0", "thread"),
+    ("2049 73 23 10 0", "rows"), ("64 784 128 10 0", "rows"),
+    ("362 123 17 50 0", "thread"), ("362 123 17 32 0", "rows"), ("257 150 131 50 0", "rows")])
 def test_mlp_form(ask, shape, form):
     assert ask([f"mlp {shape}"]) == [form]
 
